@@ -52,5 +52,12 @@ int launch_backward(const float* scores, const int* lengths, int B, int max_L1, 
                     bool precise = false, bool global = false, float* poison_value = nullptr,
                     bool* poisoned = nullptr, bool recompute = false);
 
+// Value, marginals and parameter gradients by the linear-domain sweeps (scaled.hip.h):
+// *done comes back true if they took the call, with ws.redo[b] set for the elements
+// they leave to the log-domain sweeps.  global: soft Needleman-Wunsch.
+int run_scaled(const float* scores, const int* lengths, int B, int max_L1, int max_L2, float gap,
+               float T, const Layout& ws, float* value, float* marginals, float* grad_gap,
+               float* grad_T, hipStream_t st, bool global, bool* done);
+
 }  // namespace sw
 }  // namespace d2p_amd

@@ -137,14 +137,13 @@ struct TanArgs {
     float* sdot;      // [B]: the value's tangent (G == 1)
     float* wpart;     // [B][G]: a part's tangent sum at its (max, sum) scale (G > 1)
 };
-template <bool NWG = false, bool HELP = false, bool WIDE = false, bool TAN = false>
-__global__ void __launch_bounds__(WIDE ? 2 * NW * 64 : NW * 64)
-sw_forward_kernel(const float* __restrict__ scores, const int* __restrict__ lengths,
-                  float* __restrict__ alpha_sk, float* __restrict__ brow,
-                  float* __restrict__ partition, int* __restrict__ status,
-                  uint64_t* __restrict__ fflag, float2* __restrict__ fpart, int B, int L1max,
-                  int L2max, int NSmax, float gap, float T, int R, int G, int SPW,
-                  uint32_t epoch, int ckpt, TanArgs ta) {
+template <bool NWG, bool HELP, bool WIDE, bool TAN>
+__device__ __forceinline__ void forward_sweep(const float* __restrict__ scores, const int* __restrict__ lengths,
+                                              float* __restrict__ alpha_sk, float* __restrict__ brow,
+                                              float* __restrict__ partition, int* __restrict__ status,
+                                              uint64_t* __restrict__ fflag, float2* __restrict__ fpart, int B, int L1max,
+                                              int L2max, int NSmax, float gap, float T, int R, int G, int SPW,
+                                              uint32_t epoch, int ckpt, TanArgs ta) {
     constexpr int P = PF;
     static_assert(PF == PR, "checkpoint rows are chosen per forward chunk");
     static_assert(!(TAN && WIDE), "the tangent sweep has no 16-wave form");
@@ -674,6 +673,19 @@ sw_forward_kernel(const float* __restrict__ scores, const int* __restrict__ leng
     }
 }
 
+template <bool NWG = false, bool HELP = false, bool WIDE = false, bool TAN = false>
+__global__ void __launch_bounds__(WIDE ? 2 * NW * 64 : NW * 64)
+sw_forward_kernel(const float* __restrict__ scores, const int* __restrict__ lengths,
+                  float* __restrict__ alpha_sk, float* __restrict__ brow,
+                  float* __restrict__ partition, int* __restrict__ status,
+                  uint64_t* __restrict__ fflag, float2* __restrict__ fpart, int B, int L1max,
+                  int L2max, int NSmax, float gap, float T, int R, int G, int SPW,
+                  uint32_t epoch, int ckpt, TanArgs ta) {
+    forward_sweep<NWG, HELP, WIDE, TAN>(scores, lengths, alpha_sk, brow, partition, status, fflag,
+                                        fpart, B, L1max, L2max, NSmax, gap, T, R, G, SPW, epoch,
+                                        ckpt, ta);
+}
+
 // PRECISE: accumulate dS/dgap and dS/dT per lane in double (second-order callers,
 // whose Jacobians amplify errors in these sums).
 // NWG: global alignment (/root/reference/src/nw/kernels_cpu.cpp:160-265): beta starts
@@ -690,19 +702,16 @@ sw_forward_kernel(const float* __restrict__ scores, const int* __restrict__ leng
 // RECOMP (plain variant, with HELP and WIDE): the helper waves rebuild each chunk's alpha
 // rows from a checkpoint-mode forward's stored steps (ckpt_step) instead of loading
 // them from a full table.
-template <int P, bool PRECISE = false, bool NWG = false, bool HELP = false, bool WIDE = false,
-          bool RECOMP = false>
-__global__ void __launch_bounds__(WIDE ? 2 * NW * 64 : NW * 64)
-__attribute__((amdgpu_waves_per_eu(WIDE ? 4 : 1, WIDE ? 4 : 2)))
-sw_backward_kernel(const float* __restrict__ scores, const int* __restrict__ lengths,
-                   const float* __restrict__ alpha_sk, const float* __restrict__ brow,
-                   const float* __restrict__ partition,
-                   float* __restrict__ post, float* __restrict__ grad_gap,
-                   float* __restrict__ grad_T, int* __restrict__ status, float* __restrict__ trash,
-                   uint64_t* __restrict__ bflag, float2* __restrict__ flows,
-                   double* __restrict__ bpart, float* __restrict__ poison_value, int B, int L1max,
-                   int L2max, int NSmax, float gap, float T, int R, int G, int SPW,
-                   uint32_t epoch) {
+template <int P, bool PRECISE, bool NWG, bool HELP, bool WIDE, bool RECOMP>
+__device__ __forceinline__ void backward_sweep(const float* __restrict__ scores, const int* __restrict__ lengths,
+                                               const float* __restrict__ alpha_sk, const float* __restrict__ brow,
+                                               const float* __restrict__ partition,
+                                               float* __restrict__ post, float* __restrict__ grad_gap,
+                                               float* __restrict__ grad_T, int* __restrict__ status, float* __restrict__ trash,
+                                               uint64_t* __restrict__ bflag, float2* __restrict__ flows,
+                                               double* __restrict__ bpart, float* __restrict__ poison_value, int B, int L1max,
+                                               int L2max, int NSmax, float gap, float T, int R, int G, int SPW,
+                                               uint32_t epoch) {
     extern __shared__ __align__(16) float smem[];
     __shared__ int prog[NW];
     using Acc = typename std::conditional<PRECISE, double, float>::type;
@@ -1458,6 +1467,48 @@ sw_backward_kernel(const float* __restrict__ scores, const int* __restrict__ len
     }
 }
 
+template <int P, bool PRECISE = false, bool NWG = false, bool HELP = false, bool WIDE = false,
+          bool RECOMP = false>
+__global__ void __launch_bounds__(WIDE ? 2 * NW * 64 : NW * 64)
+__attribute__((amdgpu_waves_per_eu(WIDE ? 4 : 1, WIDE ? 4 : 2)))
+sw_backward_kernel(const float* __restrict__ scores, const int* __restrict__ lengths,
+                   const float* __restrict__ alpha_sk, const float* __restrict__ brow,
+                   const float* __restrict__ partition,
+                   float* __restrict__ post, float* __restrict__ grad_gap,
+                   float* __restrict__ grad_T, int* __restrict__ status, float* __restrict__ trash,
+                   uint64_t* __restrict__ bflag, float2* __restrict__ flows,
+                   double* __restrict__ bpart, float* __restrict__ poison_value, int B, int L1max,
+                   int L2max, int NSmax, float gap, float T, int R, int G, int SPW,
+                   uint32_t epoch) {
+    backward_sweep<P, PRECISE, NWG, HELP, WIDE, RECOMP>(
+        scores, lengths, alpha_sk, brow, partition, post, grad_gap, grad_T, status, trash, bflag,
+        flows, bpart, poison_value, B, L1max, L2max, NSmax, gap, T, R, G, SPW, epoch);
+}
+
+// Both sweeps of the elements that `redo` marks (values beyond the range of the
+// linear-domain sweeps), one workgroup each; the others leave at once.  One launch, so
+// that a call without such elements, which is nearly every call, pays for one empty grid
+// (3 us) and not for two.
+template <bool NWG>
+__global__ void __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(1, 2)))
+sw_redo_kernel(const int* __restrict__ redo, const float* __restrict__ scores,
+               const int* __restrict__ lengths, const Layout ws, float* __restrict__ value,
+               float* __restrict__ post, float* __restrict__ grad_gap, float* __restrict__ grad_T,
+               int B, int L1max, int L2max, int NSmax, float gap, float T, int Rf, int Rb,
+               uint32_t epoch) {
+    int b, part;
+    split_decode(blockIdx.x, 1, b, part);
+    if (b >= B || redo[b] == 0) return;
+    forward_sweep<NWG, false, false, false>(scores, lengths, ws.alpha_sk, ws.brow, value, ws.status,
+                                            ws.fflag, ws.fpart, B, L1max, L2max, NSmax, gap, T, Rf,
+                                            1, NSmax, epoch, 0, TanArgs{});
+    __threadfence_block();
+    __syncthreads();
+    backward_sweep<8, false, NWG, false, false, false>(
+        scores, lengths, ws.alpha_sk, ws.brow, value, post, grad_gap, grad_T, ws.status, ws.trash,
+        ws.bflag, ws.flows, ws.bpart, value, B, L1max, L2max, NSmax, gap, T, Rb, 1, NSmax, epoch);
+}
+
 // grad_gap[b], grad_T[b] of a split element from the parts' sums.
 template <bool PRECISE>
 __global__ void sw_grad_merge(const double* __restrict__ bpart, const float* __restrict__ partition,
@@ -1723,6 +1774,31 @@ int launch_backward(const float* scores, const int* lengths, int B, int max_L1, 
 #undef D2P_SW_BWD
 }
 
+// LDS of the two log-domain sweeps of an unsplit element in one workgroup (8-step reverse
+// chunks, which fit longer rows than 16-step ones); the second one's static arrays come on top
+size_t redo_lds(int max_L1, int max_L2) {
+    const size_t f = lds_forward_r(ring_forward(max_L1, max_L2));
+    const size_t b = lds_backward_r(ring_backward(max_L1, max_L2), 8);
+    return (f > b ? f : b) + 1024;
+}
+
+int launch_redo(const float* scores, const int* lengths, int B, int max_L1, int max_L2, float gap,
+                float T, const Layout& ws, float* value, float* marginals, float* grad_gap,
+                float* grad_T, hipStream_t st, bool global) {
+    const size_t lds = redo_lds(max_L1, max_L2) - 1024;
+    void (*k)(const int*, const float*, const int*, const Layout, float*, float*, float*, float*,
+              int, int, int, int, float, float, int, int, uint32_t) =
+        global ? sw_redo_kernel<true> : sw_redo_kernel<false>;
+    D2P_HIP(hipFuncSetAttribute((const void*)k, hipFuncAttributeMaxDynamicSharedMemorySize,
+                                (int)lds));
+    D2P_LAUNCH(global ? "nw_redo" : "sw_redo", k, dim3(wf::split_grid(B, 1)), dim3(wf::NW * 64),
+               lds, st, ws.redo, scores, lengths, ws, value, marginals, grad_gap, grad_T, B,
+               max_L1, max_L2, (max_L1 + 63) / 64, gap, T, ring_forward(max_L1, max_L2),
+               ring_backward(max_L1, max_L2), next_epoch());
+    D2P_HIP(hipGetLastError());
+    return D2P_OK;
+}
+
 }  // namespace sw
 }  // namespace d2p_amd
 
@@ -1747,6 +1823,33 @@ extern "C" int d2p_sw_status(const void* workspace, int B, int* status, void* st
     return D2P_OK;
 }
 
+namespace {
+// Value, marginals and parameter gradients: the linear-domain sweeps where they take the
+// call, then the log-domain sweeps of the elements whose values left their range; the
+// log-domain sweeps for all elements otherwise.
+int first_order(const float* scores, const int* lengths, int B, int max_L1, int max_L2, float gap,
+                float T, const wf::Layout& ws, float* value, float* marginals, float* grad_gap,
+                float* grad_T, hipStream_t st, bool global) {
+    bool done = false;
+    if (sw::redo_lds(max_L1, max_L2) <= sw::kLdsLimit)
+        D2P_TRY(sw::run_scaled(scores, lengths, B, max_L1, max_L2, gap, T, ws, value, marginals,
+                               grad_gap, grad_T, st, global, &done));
+    if (done)
+        return sw::launch_redo(scores, lengths, B, max_L1, max_L2, gap, T, ws, value, marginals,
+                               grad_gap, grad_T, st, global);
+    const bool recompute = !global && sw::recompute_alpha(B, max_L1, max_L2, ws);
+    D2P_TRY(sw::launch_forward(scores, lengths, B, max_L1, max_L2, gap, T, ws, value, st, global,
+                               recompute));
+    bool poisoned = false;
+    D2P_TRY(sw::launch_backward(scores, lengths, B, max_L1, max_L2, gap, T, ws, value, marginals,
+                                grad_gap, grad_T, st, false, global, value, &poisoned,
+                                recompute));
+    if (poisoned) return D2P_OK;
+    return wf::launch_poison(ws.status, B, (long long)max_L1 * max_L2, marginals, nullptr, value,
+                             grad_gap, grad_T, nullptr, st);
+}
+}  // namespace
+
 extern "C" int d2p_sw_forward_marginals(const float* scores, const int* lengths, int B,
                                         int max_L1, int max_L2, float gap, float temperature,
                                         float* partition, float* marginals, float* grad_gap,
@@ -1759,18 +1862,9 @@ extern "C" int d2p_sw_forward_marginals(const float* scores, const int* lengths,
                 "null pointer argument");
     const size_t need = d2p_sw_workspace_bytes(B, max_L1, max_L2);
     D2P_REQUIRE(workspace && workspace_bytes >= need, "workspace too small");
-    hipStream_t st = (hipStream_t)stream;
     const wf::Layout ws = wf::layout(workspace, B, max_L1, max_L2, 1, true);
-    const bool recompute = sw::recompute_alpha(B, max_L1, max_L2, ws);
-    D2P_TRY(sw::launch_forward(scores, lengths, B, max_L1, max_L2, gap, temperature, ws,
-                               partition, st, false, recompute));
-    bool poisoned = false;
-    D2P_TRY(sw::launch_backward(scores, lengths, B, max_L1, max_L2, gap, temperature, ws,
-                                partition, marginals, grad_gap, grad_T, st, false, false,
-                                partition, &poisoned, recompute));
-    if (poisoned) return D2P_OK;
-    return wf::launch_poison(ws.status, B, (long long)max_L1 * max_L2, marginals, nullptr,
-                             partition, grad_gap, grad_T, nullptr, st);
+    return first_order(scores, lengths, B, max_L1, max_L2, gap, temperature, ws, partition,
+                       marginals, grad_gap, grad_T, (hipStream_t)stream, false);
 }
 
 // ---------------------------------------------------------------------------
@@ -1827,18 +1921,9 @@ extern "C" int d2p_sw_forward_marginals_noalloc(const float* scores, const int* 
     D2P_TRY(scratch_on_current_device(&ws_ptr));
     // the sweeps reset every word of the workspace they rely on (status and progress
     // words) themselves, with kernels: the previous call's contents do not matter
-    hipStream_t st = (hipStream_t)stream;
     const wf::Layout ws = wf::layout(ws_ptr, B, max_L1, max_L2, 1, true);
-    const bool recompute = sw::recompute_alpha(B, max_L1, max_L2, ws);
-    D2P_TRY(sw::launch_forward(scores, lengths, B, max_L1, max_L2, gap, temperature, ws,
-                               partition, st, false, recompute));
-    bool poisoned = false;
-    D2P_TRY(sw::launch_backward(scores, lengths, B, max_L1, max_L2, gap, temperature, ws,
-                                partition, marginals, grad_gap, grad_T, st, false, false,
-                                partition, &poisoned, recompute));
-    if (poisoned) return D2P_OK;
-    return wf::launch_poison(ws.status, B, (long long)max_L1 * max_L2, marginals, nullptr,
-                             partition, grad_gap, grad_T, nullptr, st);
+    return first_order(scores, lengths, B, max_L1, max_L2, gap, temperature, ws, partition,
+                       marginals, grad_gap, grad_T, (hipStream_t)stream, false);
 }
 
 extern "C" size_t d2p_nw_workspace_bytes(int B, int max_L1, int max_L2) {
@@ -1857,14 +1942,7 @@ extern "C" int d2p_nw_forward_marginals(const float* scores, const int* lengths,
                 "null pointer argument");
     const size_t need = d2p_nw_workspace_bytes(B, max_L1, max_L2);
     D2P_REQUIRE(workspace && workspace_bytes >= need, "workspace too small");
-    hipStream_t st = (hipStream_t)stream;
     const wf::Layout ws = wf::layout(workspace, B, max_L1, max_L2, 1, true);
-    D2P_TRY(sw::launch_forward(scores, lengths, B, max_L1, max_L2, gap, temperature, ws, value,
-                               st, true));
-    bool poisoned = false;
-    D2P_TRY(sw::launch_backward(scores, lengths, B, max_L1, max_L2, gap, temperature, ws, value,
-                                marginals, grad_gap, grad_T, st, false, true, value, &poisoned));
-    if (poisoned) return D2P_OK;
-    return wf::launch_poison(ws.status, B, (long long)max_L1 * max_L2, marginals, nullptr, value,
-                             grad_gap, grad_T, nullptr, st);
+    return first_order(scores, lengths, B, max_L1, max_L2, gap, temperature, ws, value, marginals,
+                       grad_gap, grad_T, (hipStream_t)stream, true);
 }

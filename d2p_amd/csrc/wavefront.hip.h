@@ -107,6 +107,7 @@ struct Layout {
     size_t flow_slots; // B * stripes * stored steps
     float2* fpart;     // [B][stripe] (max, scaled sum) of the partition
     double* bpart;     // [B][stripe][4] parameter-gradient sums
+    int* redo;         // [B] elements the linear-domain sweeps leave to the log-domain ones
     size_t bytes;      // bytes of this prefix
 };
 
@@ -125,6 +126,7 @@ __host__ inline Layout layout(void* workspace, int B, int max_L1, int max_L2, in
     l.flows = l.fpart = nullptr;
     l.flow_slots = 0;
     l.bpart = nullptr;
+    l.redo = nullptr;
     if (split) {
         char* p = (char*)workspace + round256(l.bytes);
         const size_t parts = (size_t)B * (ns > 0 ? ns : 1);
@@ -139,6 +141,8 @@ __host__ inline Layout layout(void* workspace, int B, int max_L1, int max_L2, in
         p += round256(parts * sizeof(float2));
         l.bpart = (double*)p;
         p += round256(parts * 4 * sizeof(double));
+        l.redo = (int*)p;
+        p += round256((size_t)B * sizeof(int));
         l.bytes = (size_t)(p - (char*)workspace);
     }
     return l;

@@ -1,0 +1,93 @@
+"""The linear-domain sweeps of soft Smith-Waterman and Needleman-Wunsch (64-bit values with
+an exponent per lane, factors 2^(c s) in 32 bits) against the double-precision oracle, at
+the edges of their stripes, chunks, parts and launch shapes, and their hand-over of
+elements whose values leave the range to the log-domain sweeps.
+
+Tolerance: a factor's relative error is delta = 2^-23 + 2^-24 max|c s| (the 32-bit 2^x, and
+the rounding of its argument).  A path of m matches multiplies m factors, whose roundings
+are independent: the logarithm of a marginal is off by some sqrt(m) delta on either side of
+a cell; four standard deviations of the two together are 8 sqrt(m) delta.
+"""
+import math
+
+import numpy as np
+import pytest
+import torch
+
+import d2p_amd
+from oracle import oracle as O
+
+pytestmark = pytest.mark.gpu
+
+# (B, L1, L2, temperature, gap, parts asked for (0: the library's choice), ragged)
+CASES = [
+    (1, 1, 1, 1.0, -1.0, 0, False),
+    (2, 63, 15, 1.0, -1.0, 0, False),      # below a stripe and a chunk
+    (2, 64, 16, 1.0, 0.0, 0, False),       # exactly one of each
+    (3, 65, 17, 0.7, -2.0, 0, False),      # one row and one column more
+    (2, 130, 1, 1.0, -1.0, 0, False),      # one column
+    (2, 1, 131, 1.0, -1.0, 0, False),      # one row
+    (9, 256, 90, 0.2, -0.5, 0, True),      # four stripes, lowest temperature taken
+    (3, 257, 66, 1.0, -1.0, 0, True),      # five stripes: two parts
+    (3, 300, 83, 1.0, -1.0, 5, True),      # parts of one stripe
+    (2, 512, 203, 3.0, 1.0, 1, True),      # eight stripes in one part, a positive gap
+    (300, 100, 45, 1.0, -1.0, 0, True),    # more elements than CUs: one reverse wave a stripe
+    (2, 600, 40, 1.0, -1.0, 1, True),      # ten stripes: parts of at most six
+    (1, 1024, 1024, 1.0, -1.0, 0, False),  # the longest taken
+]
+
+
+def _inputs(B, L1, L2, ragged):
+    g = np.random.default_rng(1000 * L1 + L2)
+    s = (1.5 * g.standard_normal((B, L1, L2))).astype(np.float32)
+    if not ragged:
+        return s, None
+    lengths = np.stack([g.integers(0, L1 + 1, B), g.integers(0, L2 + 1, B)], 1).astype(np.int32)
+    lengths[0] = L1, L2
+    lengths[-1] = 0, L2
+    return s, lengths
+
+
+def _tol(s, m, T):
+    delta = 2.0 ** -23 + 2.0 ** -24 * float(np.abs(s).max()) / T * math.log2(math.e)
+    return 8.0 * math.sqrt(m) * delta
+
+
+@pytest.mark.parametrize("nw", [False, True])
+@pytest.mark.parametrize("B,L1,L2,T,gap,parts,ragged", CASES)
+def test_scaled_sweeps_match_double_oracle(cuda, monkeypatch, B, L1, L2, T, gap, parts, ragged,
+                                           nw):
+    if parts:
+        monkeypatch.setenv("D2P_AMD_SPLIT", str(parts))
+    s, lengths = _inputs(B, L1, L2, ragged)
+    op = "soft_nw" if nw else "soft_sw"
+    lt = None if lengths is None else torch.from_numpy(lengths).to(cuda)
+    got = getattr(d2p_amd, op)(torch.from_numpy(s).to(cuda), gap, T, lengths=lt)
+    n = min(B, 9)
+    idx = list(range(n - 1)) + [B - 1]
+    want = getattr(O.get("oracle64"), op)(s[idx].astype(np.float64), gap, T,
+                                           None if lengths is None else lengths[idx])
+    tol = _tol(s, min(L1, L2), T)
+    value = got[0].cpu().numpy()[idx].astype(np.float64)
+    assert np.all(np.abs(value - want[0]) <= T * tol + 2.0 ** -23 * np.abs(want[0])), value
+    err = np.abs(got[1].cpu().numpy()[idx] - want[1]).max()
+    assert err <= tol, (err, tol)
+
+
+@pytest.mark.parametrize("nw", [False, True])
+@pytest.mark.parametrize("L1,L2", [(40, 37), (130, 70), (300, 83)])
+def test_elements_out_of_range(cuda, L1, L2, nw):
+    # element 1 has a factor beyond 32 bits: the log-domain sweeps compute it, whose
+    # rounding is that of alpha (ulp(512), over T) along the path; element 2 is masked
+    s, _ = _inputs(3, L1, L2, False)
+    s[1, L1 // 2, L2 // 2] = 300.0
+    s[2, :, L2 // 3:] = -1e30
+    op = "soft_nw" if nw else "soft_sw"
+    got = getattr(d2p_amd, op)(torch.from_numpy(s).to(cuda), -1.0, 1.0)
+    want = getattr(O.get("oracle64"), op)(s.astype(np.float64), -1.0, 1.0, None)
+    tol = _tol(np.clip(s[0], -10, 10), min(L1, L2), 1.0)
+    err = np.abs(got[1].cpu().numpy() - want[1]).max(axis=(1, 2))
+    assert err[0] <= tol and err[2] <= tol, err
+    assert err[1] <= math.sqrt(L1 + L2) * 2.0 ** -15, err
+    v = got[0].cpu().numpy().astype(np.float64)
+    assert np.all(np.abs(v - want[0]) <= 1e-5 * np.abs(want[0]) + 1e-5), (v, want[0])
