@@ -590,7 +590,7 @@ __device__ inline void poison(const Args& A, int b) {
 // ------------------------------------------------------------------ reverse sweep
 
 template <Fam F>
-__global__ void __launch_bounds__(MAXW * 64) bwd_kernel(const Args A) {
+__global__ void __launch_bounds__((Traits<F>::AFFINE ? 4 : MAXW) * 64) bwd_kernel(const Args A) {
     using Tr = Traits<F>;
     constexpr bool GLOBAL = F == NW || F == NWAFF;
     extern __shared__ __align__(16) char smem[];
@@ -1792,7 +1792,7 @@ __global__ void __launch_bounds__(256) finish_kernel(const Args A) {
     finalize<F>(A, b, L1, L2, r, bp[3]);
 }
 
-__global__ void reset_kernel(int* __restrict__ status, int* __restrict__ redo,
+static __global__ void reset_kernel(int* __restrict__ status, int* __restrict__ redo,
                              uint64_t* __restrict__ fflag, uint64_t* __restrict__ bflag, int B,
                              int G) {
     const int i = blockIdx.x * blockDim.x + threadIdx.x;
@@ -1808,10 +1808,25 @@ __global__ void reset_kernel(int* __restrict__ status, int* __restrict__ redo,
 // Parts of an element.  Parts of four stripes (a wave per SIMD) where the whole grid is
 // resident at once; else up to eight stripes in one workgroup, or parts of six and two
 // copying waves.  D2P_AMD_SPLIT=<n> asks for n parts.
+// Affine gaps: the reverse sweep keeps three states of a chunk and needs more registers
+// than two waves on a SIMD leave each other (the spilling form took 700 us at [32, 500,
+// 450], against 524 for the log-domain sweep), so a workgroup has four waves: an element
+// of up to four stripes, or parts of two and the copying waves, where all of them are
+// resident at once.  SPW = 0: neither.
+template <Fam F>
 inline Split choose_parts(int B, int ns) {
     Split sp{1, ns > 0 ? ns : 1};
     int G = 0;
     if (const char* e = getenv("D2P_AMD_SPLIT")) G = atoi(e);
+    if constexpr (Traits<F>::AFFINE) {
+        G = G < ns ? G : ns;
+        if (G <= 1 && ns <= 4) return sp;
+        G = G > (ns + 1) / 2 ? G : (ns + 1) / 2;
+        sp.SPW = (ns + G - 1) / G;
+        sp.G = (ns + sp.SPW - 1) / sp.SPW;
+        if (split_grid(B, sp.G) > device_cus()) sp.SPW = 0;
+        return sp;
+    }
     if (G <= 0) {
         const int g4 = (ns + 3) / 4;
         G = ns > 4 && split_grid(B, g4) <= device_cus() ? g4 : 1;
@@ -1858,12 +1873,12 @@ int run(Args A, void* table, size_t table_bytes, bool* done, hipStream_t st, con
     using Tr = Traits<F>;
     *done = false;
     const int ns = (A.L1max + 63) / 64;
-    const Split sp = choose_parts(A.B, ns);
+    const Split sp = choose_parts<F>(A.B, ns);
     A.NSmax = ns;
     A.G = sp.G;
     A.SPW = sp.SPW;
     A.mem = carve<F>(table, A.B, A.L1max, A.L2max, sp.G);
-    if (ns == 0 || A.L2max == 0 || A.mem.bytes > table_bytes) return D2P_OK;
+    if (ns == 0 || A.L2max == 0 || sp.SPW == 0 || A.mem.bytes > table_bytes) return D2P_OK;
     A.epoch = next_epoch();
     const int copying = sp.G > 1 ? 2 : 0;
     if (sp.G > 1)

@@ -72,14 +72,17 @@ __device__ __forceinline__ float lse4(float a, float b, float x, float y, float 
 // planes of each chunk's alphas to the table once wave l has finished the chunk:
 // wave l leaves them in a tile of the helper's (its own buffer for even chunks, a
 // region after the rings for odd ones) and stores only the D plane itself.
-template <bool NWA = false, bool HELP = false>
-__global__ void __launch_bounds__(NW * 64)
-swa_forward_kernel(const float* __restrict__ scores, const int* __restrict__ lengths,
-                   float* __restrict__ alpha_sk, float* __restrict__ brow,
-                   float* __restrict__ partition, int* __restrict__ status,
-                   uint64_t* __restrict__ fflag, float2* __restrict__ fpart, int B, int L1max,
-                   int L2max, int NSmax, float go, float ge, float T, int R, int G, int SPW,
-                   uint32_t epoch) {
+template <bool NWA, bool HELP>
+__device__ __forceinline__ void forward_sweep(const float* __restrict__ scores,
+                                              const int* __restrict__ lengths,
+                                              float* __restrict__ alpha_sk,
+                                              float* __restrict__ brow,
+                                              float* __restrict__ partition,
+                                              int* __restrict__ status,
+                                              uint64_t* __restrict__ fflag,
+                                              float2* __restrict__ fpart, int B, int L1max,
+                                              int L2max, int NSmax, float go, float ge, float T,
+                                              int R, int G, int SPW, uint32_t epoch) {
     constexpr int P = PF;
     static_assert(!HELP || !NWA, "helper waves serve the local form");
     extern __shared__ __align__(16) float smem[];
@@ -408,6 +411,18 @@ swa_forward_kernel(const float* __restrict__ scores, const int* __restrict__ len
     }
 }
 
+template <bool NWA = false, bool HELP = false>
+__global__ void __launch_bounds__(NW * 64)
+swa_forward_kernel(const float* __restrict__ scores, const int* __restrict__ lengths,
+                   float* __restrict__ alpha_sk, float* __restrict__ brow,
+                   float* __restrict__ partition, int* __restrict__ status,
+                   uint64_t* __restrict__ fflag, float2* __restrict__ fpart, int B, int L1max,
+                   int L2max, int NSmax, float go, float ge, float T, int R, int G, int SPW,
+                   uint32_t epoch) {
+    forward_sweep<NWA, HELP>(scores, lengths, alpha_sk, brow, partition, status, fflag, fpart, B,
+                             L1max, L2max, NSmax, go, ge, T, R, G, SPW, epoch);
+}
+
 // NWA: global alignment (/root/reference/src/nw_affine/kernels_cpu.cpp:193-347): beta
 // starts at the terminal cell only, with the weights of its three states; every state
 // has three candidates (I and D also take D above / I to the left with an open), so
@@ -421,17 +436,23 @@ swa_forward_kernel(const float* __restrict__ scores, const int* __restrict__ len
 // (publishing hprog[q] = chunks loaded), writes the chunk's output tile out once
 // wave q has finished the chunk (prog[q]), and then loads chunk k + 2 into that
 // buffer.  Wave q loads only its rows above and flows.
-template <bool NWA = false, bool HELP = false>
-__global__ void __launch_bounds__(NW * 64)
-swa_backward_kernel(const float* __restrict__ scores, const int* __restrict__ lengths,
-                    const float* __restrict__ alpha_sk, const float* __restrict__ brow,
-                    const float* __restrict__ partition, float* __restrict__ post,
-                    float* __restrict__ grad_open, float* __restrict__ grad_ext,
-                    float* __restrict__ grad_T, int* __restrict__ status,
-                    float* __restrict__ trash, uint64_t* __restrict__ bflag,
-                    float4* __restrict__ flows4, float* __restrict__ flows1,
-                    double* __restrict__ bpart, int B, int L1max, int L2max, int NSmax, float go,
-                    float ge, float T, int R, int G, int SPW, uint32_t epoch) {
+template <bool NWA, bool HELP>
+__device__ __forceinline__ void backward_sweep(const float* __restrict__ scores,
+                                               const int* __restrict__ lengths,
+                                               const float* __restrict__ alpha_sk,
+                                               const float* __restrict__ brow,
+                                               const float* __restrict__ partition,
+                                               float* __restrict__ post,
+                                               float* __restrict__ grad_open,
+                                               float* __restrict__ grad_ext,
+                                               float* __restrict__ grad_T,
+                                               int* __restrict__ status, float* __restrict__ trash,
+                                               uint64_t* __restrict__ bflag,
+                                               float4* __restrict__ flows4,
+                                               float* __restrict__ flows1,
+                                               double* __restrict__ bpart, int B, int L1max,
+                                               int L2max, int NSmax, float go, float ge, float T,
+                                               int R, int G, int SPW, uint32_t epoch) {
     constexpr int P = PB;
     static_assert(!HELP || !NWA, "helper waves move quad tiles");
     extern __shared__ __align__(16) float smem[];
@@ -1022,6 +1043,56 @@ swa_backward_kernel(const float* __restrict__ scores, const int* __restrict__ le
     }
 }
 
+template <bool NWA = false, bool HELP = false>
+__global__ void __launch_bounds__(NW * 64)
+swa_backward_kernel(const float* __restrict__ scores, const int* __restrict__ lengths,
+                    const float* __restrict__ alpha_sk, const float* __restrict__ brow,
+                    const float* __restrict__ partition, float* __restrict__ post,
+                    float* __restrict__ grad_open, float* __restrict__ grad_ext,
+                    float* __restrict__ grad_T, int* __restrict__ status,
+                    float* __restrict__ trash, uint64_t* __restrict__ bflag,
+                    float4* __restrict__ flows4, float* __restrict__ flows1,
+                    double* __restrict__ bpart, int B, int L1max, int L2max, int NSmax, float go,
+                    float ge, float T, int R, int G, int SPW, uint32_t epoch) {
+    backward_sweep<NWA, HELP>(scores, lengths, alpha_sk, brow, partition, post, grad_open,
+                              grad_ext, grad_T, status, trash, bflag, flows4, flows1, bpart, B,
+                              L1max, L2max, NSmax, go, ge, T, R, G, SPW, epoch);
+}
+
+// Both sweeps of the elements that `redo` marks (values beyond the range of the
+// linear-domain sweeps), one workgroup each; the others leave at once.
+template <bool NWA>
+__global__ void __launch_bounds__(NW * 64)
+swa_redo_kernel(const int* __restrict__ redo, const float* __restrict__ scores,
+                const int* __restrict__ lengths, const Layout ws, float* __restrict__ value,
+                float* __restrict__ post, float* __restrict__ grad_open,
+                float* __restrict__ grad_ext, float* __restrict__ grad_T, int B, int L1max,
+                int L2max, int NSmax, float go, float ge, float T, int Rf, int Rb,
+                uint32_t epoch) {
+    __shared__ int poison_flag;
+    int b, part;
+    split_decode(blockIdx.x, 1, b, part);
+    if (b >= B || redo[b] == 0) return;
+    forward_sweep<NWA, false>(scores, lengths, ws.alpha_sk, ws.brow, value, ws.status, ws.fflag,
+                              ws.fpart, B, L1max, L2max, NSmax, go, ge, T, Rf, 1, NSmax, epoch);
+    __threadfence_block();
+    __syncthreads();
+    backward_sweep<NWA, false>(scores, lengths, ws.alpha_sk, ws.brow, value, post, grad_open,
+                               grad_ext, grad_T, ws.status, ws.trash, ws.bflag,
+                               reinterpret_cast<float4*>(ws.flows), nullptr, ws.bpart, B, L1max,
+                               L2max, NSmax, go, ge, T, Rb, 1, NSmax, epoch);
+    // waits that gave up: NaN everywhere
+    wait_vmcnt<0>();
+    __syncthreads();
+    if (threadIdx.x == 0) poison_flag = load_status(ws.status + b);
+    __syncthreads();
+    if (poison_flag == 0) return;
+    const float nan = __builtin_nanf("");
+    const size_t n = (size_t)L1max * L2max;
+    for (size_t i = threadIdx.x; i < n; i += blockDim.x) post[(size_t)b * n + i] = nan;
+    if (threadIdx.x == 0) value[b] = grad_open[b] = grad_ext[b] = grad_T[b] = nan;
+}
+
 // grad_open[b], grad_ext[b], grad_T[b] of a split element from the parts' sums.
 __global__ void swa_grad_merge(const double* __restrict__ bpart, const float* __restrict__ partition,
                                float* __restrict__ grad_open, float* __restrict__ grad_ext,
@@ -1165,6 +1236,29 @@ int launch_backward(const float* scores, const int* lengths, int B, int max_L1, 
     return D2P_OK;
 }
 
+// LDS of the two log-domain sweeps of an unsplit element in one workgroup (the second
+// one's static arrays come on top)
+size_t redo_lds(int max_L1, int max_L2, bool nwa) {
+    const size_t f = lds_forward_r(ring_forward(max_L1, max_L2));
+    const size_t b = lds_backward_r(ring_backward(max_L1, max_L2), nwa);
+    return (f > b ? f : b) + 1024;
+}
+
+int launch_redo(const float* scores, const int* lengths, int B, int max_L1, int max_L2, float go,
+                float ge, float T, const Layout& ws, float* value, float* marginals,
+                float* grad_open, float* grad_ext, float* grad_T, hipStream_t st, bool nwa) {
+    const size_t lds = redo_lds(max_L1, max_L2, nwa) - 1024;
+    auto k = nwa ? swa_redo_kernel<true> : swa_redo_kernel<false>;
+    D2P_HIP(hipFuncSetAttribute((const void*)k, hipFuncAttributeMaxDynamicSharedMemorySize,
+                                (int)lds));
+    D2P_LAUNCH(nwa ? "nwa_redo" : "swa_redo", k, dim3(split_grid(B, 1)), dim3(NW * 64), lds, st,
+               ws.redo, scores, lengths, ws, value, marginals, grad_open, grad_ext, grad_T, B,
+               max_L1, max_L2, (max_L1 + 63) / 64, go, ge, T, ring_forward(max_L1, max_L2),
+               ring_backward(max_L1, max_L2), next_epoch());
+    D2P_HIP(hipGetLastError());
+    return D2P_OK;
+}
+
 }  // namespace swa
 }  // namespace d2p_amd
 
@@ -1192,6 +1286,13 @@ int affine_forward_marginals(const float* scores, const int* lengths, int B, int
     D2P_REQUIRE(workspace && workspace_bytes >= need, "workspace too small");
     hipStream_t st = (hipStream_t)stream;
     const wf::Layout ws = swa::affine_layout(workspace, B, max_L1, max_L2, true);
+    bool done = false;
+    if (swa::redo_lds(max_L1, max_L2, nwa) <= swa::kLdsLimit)
+        D2P_TRY(swa::run_scaled(scores, lengths, B, max_L1, max_L2, gap_open, gap_ext, temperature,
+                                ws, value, marginals, grad_open, grad_ext, grad_T, st, nwa, &done));
+    if (done)
+        return swa::launch_redo(scores, lengths, B, max_L1, max_L2, gap_open, gap_ext, temperature,
+                                ws, value, marginals, grad_open, grad_ext, grad_T, st, nwa);
     D2P_TRY(swa::launch_forward(scores, lengths, B, max_L1, max_L2, gap_open, gap_ext,
                                 temperature, ws, value, st, nwa));
     D2P_TRY(swa::launch_backward(scores, lengths, B, max_L1, max_L2, gap_open, gap_ext,

@@ -75,16 +75,38 @@ def test_scaled_sweeps_match_double_oracle(cuda, monkeypatch, B, L1, L2, T, gap,
 
 
 @pytest.mark.parametrize("nw", [False, True])
+@pytest.mark.parametrize("B,L1,L2,T,gap,parts,ragged", CASES)
+def test_scaled_affine_sweeps_match_double_oracle(cuda, monkeypatch, B, L1, L2, T, gap, parts,
+                                                  ragged, nw):
+    if parts:
+        monkeypatch.setenv("D2P_AMD_SPLIT", str(parts))
+    s, lengths = _inputs(B, L1, L2, ragged)
+    op = "soft_nw_affine" if nw else "soft_sw_affine"
+    lt = None if lengths is None else torch.from_numpy(lengths).to(cuda)
+    got = getattr(d2p_amd, op)(torch.from_numpy(s).to(cuda), gap - 1.0, gap / 2, T, lengths=lt)
+    n = min(B, 9)
+    idx = list(range(n - 1)) + [B - 1]
+    want = getattr(O.get("oracle64"), op)(s[idx].astype(np.float64), gap - 1.0, gap / 2, T,
+                                          None if lengths is None else lengths[idx])
+    tol = _tol(s, min(L1, L2), T)
+    value = got[0].cpu().numpy()[idx].astype(np.float64)
+    assert np.all(np.abs(value - want[0]) <= T * tol + 2.0 ** -23 * np.abs(want[0])), value
+    err = np.abs(got[1].cpu().numpy()[idx] - want[1]).max()
+    assert err <= tol, (err, tol)
+
+
+@pytest.mark.parametrize("op,gaps", [("soft_sw", (-1.0,)), ("soft_nw", (-1.0,)),
+                                     ("soft_sw_affine", (-2.0, -0.5)),
+                                     ("soft_nw_affine", (-2.0, -0.5))])
 @pytest.mark.parametrize("L1,L2", [(40, 37), (130, 70), (300, 83)])
-def test_elements_out_of_range(cuda, L1, L2, nw):
+def test_elements_out_of_range(cuda, L1, L2, op, gaps):
     # element 1 has a factor beyond 32 bits: the log-domain sweeps compute it, whose
     # rounding is that of alpha (ulp(512), over T) along the path; element 2 is masked
     s, _ = _inputs(3, L1, L2, False)
     s[1, L1 // 2, L2 // 2] = 300.0
     s[2, :, L2 // 3:] = -1e30
-    op = "soft_nw" if nw else "soft_sw"
-    got = getattr(d2p_amd, op)(torch.from_numpy(s).to(cuda), -1.0, 1.0)
-    want = getattr(O.get("oracle64"), op)(s.astype(np.float64), -1.0, 1.0, None)
+    got = getattr(d2p_amd, op)(torch.from_numpy(s).to(cuda), *gaps, 1.0)
+    want = getattr(O.get("oracle64"), op)(s.astype(np.float64), *gaps, 1.0, None)
     tol = _tol(np.clip(s[0], -10, 10), min(L1, L2), 1.0)
     err = np.abs(got[1].cpu().numpy() - want[1]).max(axis=(1, 2))
     assert err[0] <= tol and err[2] <= tol, err
