@@ -1807,12 +1807,14 @@ static __global__ void reset_kernel(int* __restrict__ status, int* __restrict__ 
 
 // Parts of an element.  Parts of four stripes (a wave per SIMD) where the whole grid is
 // resident at once; else up to eight stripes in one workgroup, or parts of six and two
-// copying waves.  D2P_AMD_SPLIT=<n> asks for n parts.
+// copying waves if those are resident.  SPW = 0: none of these; parts that run one after
+// another lose to the log-domain sweeps' resident parts of eight (SW [128, 1024, 512],
+// forward and backward: 806 against 621 us).  D2P_AMD_SPLIT=<n> asks for n parts.
 // Affine gaps: the reverse sweep keeps three states of a chunk and needs more registers
 // than two waves on a SIMD leave each other (the spilling form took 700 us at [32, 500,
 // 450], against 524 for the log-domain sweep), so a workgroup has four waves: an element
 // of up to four stripes, or parts of two and the copying waves, where all of them are
-// resident at once.  SPW = 0: neither.
+// resident at once.
 template <Fam F>
 inline Split choose_parts(int B, int ns) {
     Split sp{1, ns > 0 ? ns : 1};
@@ -1837,6 +1839,7 @@ inline Split choose_parts(int B, int ns) {
     G = G > g6 ? G : g6;
     sp.SPW = (ns + G - 1) / G;
     sp.G = (ns + sp.SPW - 1) / sp.SPW;
+    if (split_grid(B, sp.G) > device_cus()) sp.SPW = 0;
     return sp;
 }
 
