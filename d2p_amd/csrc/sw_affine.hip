@@ -25,6 +25,7 @@
 #include <cstdlib>
 #include <type_traits>
 
+#include "scaled_sweeps.hip.h"
 #include "wavefront.hip.h"
 #include "../../include/d2p_amd.h"
 #include "capi_util.hip.h"
@@ -1059,11 +1060,12 @@ swa_backward_kernel(const float* __restrict__ scores, const int* __restrict__ le
                               L1max, L2max, NSmax, go, ge, T, R, G, SPW, epoch);
 }
 
-// Both sweeps of the elements that `redo` marks (values beyond the range of the
-// linear-domain sweeps), one workgroup each; the others leave at once.
+// After the linear-domain sweeps: the end of split elements, then both log-domain sweeps
+// of the elements that `redo` marks (values out of range), one workgroup each; the
+// others leave at once.
 template <bool NWA>
 __global__ void __launch_bounds__(NW * 64)
-swa_redo_kernel(const int* __restrict__ redo, const float* __restrict__ scores,
+swa_redo_kernel(const sc::Args A, const float* __restrict__ scores,
                 const int* __restrict__ lengths, const Layout ws, float* __restrict__ value,
                 float* __restrict__ post, float* __restrict__ grad_open,
                 float* __restrict__ grad_ext, float* __restrict__ grad_T, int B, int L1max,
@@ -1072,7 +1074,10 @@ swa_redo_kernel(const int* __restrict__ redo, const float* __restrict__ scores,
     __shared__ int poison_flag;
     int b, part;
     split_decode(blockIdx.x, 1, b, part);
-    if (b >= B || redo[b] == 0) return;
+    if (b >= B) return;
+    sc::finish_element<NWA ? sc::NWAFF : sc::AFF>(A, b);
+    if (A.redo[b] == 0) return;
+    __syncthreads();
     forward_sweep<NWA, false>(scores, lengths, ws.alpha_sk, ws.brow, value, ws.status, ws.fflag,
                               ws.fpart, B, L1max, L2max, NSmax, go, ge, T, Rf, 1, NSmax, epoch);
     __threadfence_block();
@@ -1244,7 +1249,7 @@ size_t redo_lds(int max_L1, int max_L2, bool nwa) {
     return (f > b ? f : b) + 1024;
 }
 
-int launch_redo(const float* scores, const int* lengths, int B, int max_L1, int max_L2, float go,
+int launch_redo(const sc::Args& args, const float* scores, const int* lengths, int B, int max_L1, int max_L2, float go,
                 float ge, float T, const Layout& ws, float* value, float* marginals,
                 float* grad_open, float* grad_ext, float* grad_T, hipStream_t st, bool nwa) {
     const size_t lds = redo_lds(max_L1, max_L2, nwa) - 1024;
@@ -1252,7 +1257,7 @@ int launch_redo(const float* scores, const int* lengths, int B, int max_L1, int 
     D2P_HIP(hipFuncSetAttribute((const void*)k, hipFuncAttributeMaxDynamicSharedMemorySize,
                                 (int)lds));
     D2P_LAUNCH(nwa ? "nwa_redo" : "swa_redo", k, dim3(split_grid(B, 1)), dim3(NW * 64), lds, st,
-               ws.redo, scores, lengths, ws, value, marginals, grad_open, grad_ext, grad_T, B,
+               args, scores, lengths, ws, value, marginals, grad_open, grad_ext, grad_T, B,
                max_L1, max_L2, (max_L1 + 63) / 64, go, ge, T, ring_forward(max_L1, max_L2),
                ring_backward(max_L1, max_L2), next_epoch());
     D2P_HIP(hipGetLastError());
@@ -1287,11 +1292,13 @@ int affine_forward_marginals(const float* scores, const int* lengths, int B, int
     hipStream_t st = (hipStream_t)stream;
     const wf::Layout ws = swa::affine_layout(workspace, B, max_L1, max_L2, true);
     bool done = false;
+    sc::Args args;
     if (swa::redo_lds(max_L1, max_L2, nwa) <= swa::kLdsLimit)
         D2P_TRY(swa::run_scaled(scores, lengths, B, max_L1, max_L2, gap_open, gap_ext, temperature,
-                                ws, value, marginals, grad_open, grad_ext, grad_T, st, nwa, &done));
+                                ws, value, marginals, grad_open, grad_ext, grad_T, st, nwa, &done,
+                                &args));
     if (done)
-        return swa::launch_redo(scores, lengths, B, max_L1, max_L2, gap_open, gap_ext, temperature,
+        return swa::launch_redo(args, scores, lengths, B, max_L1, max_L2, gap_open, gap_ext, temperature,
                                 ws, value, marginals, grad_open, grad_ext, grad_T, st, nwa);
     D2P_TRY(swa::launch_forward(scores, lengths, B, max_L1, max_L2, gap_open, gap_ext,
                                 temperature, ws, value, st, nwa));

@@ -4,6 +4,7 @@
 #include <hip/hip_runtime.h>
 #include <stddef.h>
 
+#include "scaled.hip.h"
 #include "wavefront.hip.h"
 
 namespace d2p_amd {
@@ -54,10 +55,11 @@ int launch_backward(const float* scores, const int* lengths, int B, int max_L1, 
 
 // Value, marginals and parameter gradients by the linear-domain sweeps (scaled.hip.h):
 // *done comes back true if they took the call, with ws.redo[b] set for the elements
-// they leave to the log-domain sweeps.  global: soft Needleman-Wunsch.
+// they leave to the log-domain sweeps, and with *args for sc::finish_element, which ends
+// split elements.  global: soft Needleman-Wunsch.
 int run_scaled(const float* scores, const int* lengths, int B, int max_L1, int max_L2, float gap,
                float T, const Layout& ws, float* value, float* marginals, float* grad_gap,
-               float* grad_T, hipStream_t st, bool global, bool* done);
+               float* grad_T, hipStream_t st, bool global, bool* done, sc::Args* args);
 
 }  // namespace sw
 }  // namespace d2p_amd

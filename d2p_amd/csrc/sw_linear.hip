@@ -23,6 +23,7 @@
 #include <type_traits>
 #include <vector>
 
+#include "scaled_sweeps.hip.h"
 #include "wavefront.hip.h"
 #include "../../include/d2p_amd.h"
 #include "capi_util.hip.h"
@@ -1485,20 +1486,23 @@ sw_backward_kernel(const float* __restrict__ scores, const int* __restrict__ len
         flows, bpart, poison_value, B, L1max, L2max, NSmax, gap, T, R, G, SPW, epoch);
 }
 
-// Both sweeps of the elements that `redo` marks (values beyond the range of the
-// linear-domain sweeps), one workgroup each; the others leave at once.  One launch, so
-// that a call without such elements, which is nearly every call, pays for one empty grid
+// After the linear-domain sweeps: the end of split elements, then both log-domain sweeps
+// of the elements that `redo` marks (values out of range), one workgroup each; the
+// others leave at once.  One launch, so that a call without such elements, which is nearly every call, pays for one empty grid
 // (3 us) and not for two.
 template <bool NWG>
 __global__ void __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(1, 2)))
-sw_redo_kernel(const int* __restrict__ redo, const float* __restrict__ scores,
+sw_redo_kernel(const sc::Args A, const float* __restrict__ scores,
                const int* __restrict__ lengths, const Layout ws, float* __restrict__ value,
                float* __restrict__ post, float* __restrict__ grad_gap, float* __restrict__ grad_T,
                int B, int L1max, int L2max, int NSmax, float gap, float T, int Rf, int Rb,
                uint32_t epoch) {
     int b, part;
     split_decode(blockIdx.x, 1, b, part);
-    if (b >= B || redo[b] == 0) return;
+    if (b >= B) return;
+    sc::finish_element<NWG ? sc::NW : sc::SW>(A, b);
+    if (A.redo[b] == 0) return;
+    __syncthreads();
     forward_sweep<NWG, false, false, false>(scores, lengths, ws.alpha_sk, ws.brow, value, ws.status,
                                             ws.fflag, ws.fpart, B, L1max, L2max, NSmax, gap, T, Rf,
                                             1, NSmax, epoch, 0, TanArgs{});
@@ -1783,17 +1787,17 @@ size_t redo_lds(int max_L1, int max_L2) {
     return (f > b ? f : b) + 1024;
 }
 
-int launch_redo(const float* scores, const int* lengths, int B, int max_L1, int max_L2, float gap,
+int launch_redo(const sc::Args& args, const float* scores, const int* lengths, int B, int max_L1, int max_L2, float gap,
                 float T, const Layout& ws, float* value, float* marginals, float* grad_gap,
                 float* grad_T, hipStream_t st, bool global) {
     const size_t lds = redo_lds(max_L1, max_L2) - 1024;
-    void (*k)(const int*, const float*, const int*, const Layout, float*, float*, float*, float*,
+    void (*k)(const sc::Args, const float*, const int*, const Layout, float*, float*, float*, float*,
               int, int, int, int, float, float, int, int, uint32_t) =
         global ? sw_redo_kernel<true> : sw_redo_kernel<false>;
     D2P_HIP(hipFuncSetAttribute((const void*)k, hipFuncAttributeMaxDynamicSharedMemorySize,
                                 (int)lds));
     D2P_LAUNCH(global ? "nw_redo" : "sw_redo", k, dim3(wf::split_grid(B, 1)), dim3(wf::NW * 64),
-               lds, st, ws.redo, scores, lengths, ws, value, marginals, grad_gap, grad_T, B,
+               lds, st, args, scores, lengths, ws, value, marginals, grad_gap, grad_T, B,
                max_L1, max_L2, (max_L1 + 63) / 64, gap, T, ring_forward(max_L1, max_L2),
                ring_backward(max_L1, max_L2), next_epoch());
     D2P_HIP(hipGetLastError());
@@ -1832,11 +1836,12 @@ int first_order(const float* scores, const int* lengths, int B, int max_L1, int 
                 float T, const wf::Layout& ws, float* value, float* marginals, float* grad_gap,
                 float* grad_T, hipStream_t st, bool global) {
     bool done = false;
+    sc::Args args;
     if (sw::redo_lds(max_L1, max_L2) <= sw::kLdsLimit)
         D2P_TRY(sw::run_scaled(scores, lengths, B, max_L1, max_L2, gap, T, ws, value, marginals,
-                               grad_gap, grad_T, st, global, &done));
+                               grad_gap, grad_T, st, global, &done, &args));
     if (done)
-        return sw::launch_redo(scores, lengths, B, max_L1, max_L2, gap, T, ws, value, marginals,
+        return sw::launch_redo(args, scores, lengths, B, max_L1, max_L2, gap, T, ws, value, marginals,
                                grad_gap, grad_T, st, global);
     const bool recompute = !global && sw::recompute_alpha(B, max_L1, max_L2, ws);
     D2P_TRY(sw::launch_forward(scores, lengths, B, max_L1, max_L2, gap, T, ws, value, st, global,

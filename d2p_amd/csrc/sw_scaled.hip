@@ -8,10 +8,12 @@ namespace sw {
 
 int run_scaled(const float* scores, const int* lengths, int B, int max_L1, int max_L2, float gap,
                float T, const Layout& ws, float* value, float* marginals, float* grad_gap,
-               float* grad_T, hipStream_t st, bool global, bool* done) {
+               float* grad_T, hipStream_t st, bool global, bool* done,
+               sc::Args* args) {
     *done = false;
     if (!sc::takes(max_L1, max_L2, T, gap, 0.0)) return D2P_OK;
-    sc::Args A{};
+    sc::Args& A = *args;
+    A = sc::Args{};
     A.m = scores;
     A.lengths = lengths;
     A.out = marginals;

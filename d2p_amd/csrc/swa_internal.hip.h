@@ -3,6 +3,7 @@
 #pragma once
 #include <hip/hip_runtime.h>
 
+#include "scaled.hip.h"
 #include "wavefront.hip.h"
 
 namespace d2p_amd {
@@ -30,11 +31,12 @@ int launch_backward(const float* scores, const int* lengths, int B, int max_L1, 
 
 // Value, marginals and parameter gradients by the linear-domain sweeps (scaled.hip.h):
 // *done comes back true if they took the call, with ws.redo[b] set for the elements
-// they leave to the log-domain sweeps.
+// they leave to the log-domain sweeps, and with *args for sc::finish_element, which ends
+// split elements.
 int run_scaled(const float* scores, const int* lengths, int B, int max_L1, int max_L2, float go,
                float ge, float T, const Layout& ws, float* value, float* marginals,
                float* grad_open, float* grad_ext, float* grad_T, hipStream_t st, bool nwa,
-               bool* done);
+               bool* done, sc::Args* args);
 
 }  // namespace swa
 }  // namespace d2p_amd

@@ -9,10 +9,12 @@ namespace swa {
 int run_scaled(const float* scores, const int* lengths, int B, int max_L1, int max_L2, float go,
                float ge, float T, const Layout& ws, float* value, float* marginals,
                float* grad_open, float* grad_ext, float* grad_T, hipStream_t st, bool nwa,
-               bool* done) {
+               bool* done,
+               sc::Args* args) {
     *done = false;
     if (!sc::takes(max_L1, max_L2, T, go, ge)) return D2P_OK;
-    sc::Args A{};
+    sc::Args& A = *args;
+    A = sc::Args{};
     A.m = scores;
     A.lengths = lengths;
     A.out = marginals;

@@ -141,8 +141,8 @@ __host__ inline Layout layout(void* workspace, int B, int max_L1, int max_L2, in
         p += round256(parts * sizeof(float2));
         l.bpart = (double*)p;
         p += round256(parts * 4 * sizeof(double));
-        l.redo = (int*)p;
-        p += round256((size_t)B * sizeof(int));
+        // (fpart is used by split log-domain sweeps only, redo by the others)
+        l.redo = (int*)l.fpart;
         l.bytes = (size_t)(p - (char*)workspace);
     }
     return l;
