@@ -35,10 +35,16 @@ using namespace wf;
 
 constexpr int DUMMY = 64 + PF;       // per-wave LDS sink for the lanes that do not publish
 
-// HELP (costs from memory, unbanded, at most NW/2 stripes per part): wave NW/2 + l
+// HELP (costs from memory, at most NW/2 stripes per part): wave NW/2 + l
 // loads stripe l's cost chunks one chunk ahead into wave l's tiles (cprog[l] = chunks
 // loaded) and writes each chunk's alpha rows to the table from a tile in its own,
 // otherwise unused, buffers once wave l has finished the chunk.
+//
+// A band makes the stripes a chain, nine chunks of one after nine of another, whose time is
+// the sweeping wave's instructions per chunk.  At [16, 4096, 4096], bandwidth 64: 1.78 ms
+// without helpers and with the band test on every cell's column, 1.26 ms with helpers
+// and each row's cells as an interval of steps (band_columns).  (The interval also
+// replaces the column test without a band: [512, 256, 256] 105 -> 100 us.)
 template <bool HELP = false>
 __global__ void __launch_bounds__(NW * 64)
 dtw_forward_kernel(const float* __restrict__ costs, const int* __restrict__ lengths,
@@ -109,7 +115,7 @@ dtw_forward_kernel(const float* __restrict__ costs, const int* __restrict__ leng
     }
 
     if constexpr (HELP) {
-        if (NL > NW / 2 || bandwidth >= 0) {   // never: the host picks HELP for these only
+        if (NL > NW / 2) {   // never: the host picks HELP for parts of at most NW/2
             if (threadIdx.x == 0) atomicOr(st, 2);
             return;
         }
@@ -117,7 +123,12 @@ dtw_forward_kernel(const float* __restrict__ costs, const int* __restrict__ leng
         if (l >= 0 && l < NL) {
             const int s = s_begin + l;
             const int i0 = s * 64;
-            // unbanded: the window is every chunk and the table starts at step 0
+            // the stripe's window, where its table starts
+            int t_lo, t_hi;
+            band_window(s, L1, L2, bw, t_lo, t_hi);
+            const int k_lo =
+                __builtin_amdgcn_readfirstlane(t_lo <= t_hi ? min(t_lo / P, nch) : nch);
+            const int k_end = __builtin_amdgcn_readfirstlane(t_lo <= t_hi ? t_hi / P + 1 : nch);
             float* out = band_stripe(alpha_sk, b, elem_steps, s, stride) + APAD * 64;
             const uint32_t ltiles = lds_address(smem + l * WBUF);   // wave l's cost tiles
             const float* atiles = smem + wave * WBUF;               // its alpha tiles
@@ -125,25 +136,25 @@ dtw_forward_kernel(const float* __restrict__ costs, const int* __restrict__ leng
                 dma_tile<P, 1>(ltiles + (k & 1) * Tile::FLOATS * 4, cbase, i0, L1max, L2max,
                                lane, k * P);
             };
-            if (nch > 0) {
-                load(0);
+            if (k_lo < k_end) {
+                load(k_lo);
                 wait_vmcnt<0>();
-                publish(cprog, l, 1);
-                if (nch > 1) load(1);
+                publish(cprog, l, k_lo + 1);
+                if (k_lo + 1 < k_end) load(k_lo + 1);
             }
-            for (int k = 0; k < nch; ++k) {
-                if (k + 1 < nch) {
-                    // chunk k + 1's loads: the last issued at k = 0, else followed by the
-                    // P/4 alpha stores of chunk k - 1
-                    if (k == 0) wait_vmcnt<0>(); else wait_vmcnt<P / 4>();
+            for (int k = k_lo; k < k_end; ++k) {
+                if (k + 1 < k_end) {
+                    // chunk k + 1's loads: the last issued at k = k_lo, else followed by
+                    // the P/4 alpha stores of chunk k - 1
+                    if (k == k_lo) wait_vmcnt<0>(); else wait_vmcnt<P / 4>();
                     publish(cprog, l, k + 2);   // also completes this wave's LDS reads
                 }
                 // once wave l has finished chunk k, its cost tile k & 1 takes chunk k + 2
                 // and its alpha rows (alpha tile k & 1) go to the table
                 wait_for(prog, l, l * PROG_STRIDE + k + 1, st);
-                if (k + 2 < nch) load(k + 2);
+                if (k + 2 < k_end) load(k + 2);
                 const float* at = atiles + (k & 1) * Tile::FLOATS;
-                float* dst = out + (size_t)k * P * 64;
+                float* dst = out + (size_t)(k - k_lo) * P * 64;
 #pragma unroll
                 for (int i = 0; i < P / 4; ++i) {
                     const float4 v = *reinterpret_cast<const float4*>(at + 256 * i + 4 * lane);
@@ -156,8 +167,11 @@ dtw_forward_kernel(const float* __restrict__ costs, const int* __restrict__ leng
     for (int l = wave; l < NL; l += NW) {
         const int s = s_begin + l;
         const int i0 = s * 64;
-        const int L2eff = (i0 + lane < L1) ? L2 : 0;   // rows past L1 are never valid
-        const float ej = band_centre(i0 + lane + 1, L1, L2);
+        // the row's valid cells: steps t_row .. t_row + cells - 1 (rows past L1: none)
+        int t_row, cells;
+        band_columns(band_centre(i0 + lane + 1, L1, L2), bw, (i0 + lane < L1) ? L2 : 0, t_row,
+                     cells);
+        t_row += lane;
         const bool last_row = i0 + lane == L1 - 1;
         const float* ring_in = ring_from(rings, l, R);
         float* ring_out = ring_of(rings, l, R);
@@ -264,6 +278,7 @@ dtw_forward_kernel(const float* __restrict__ costs, const int* __restrict__ leng
             // k & 1 (written to the table by the helper, which has written that tile's
             // previous chunk before publishing this chunk's costs as loaded)
             float* atile = smem + (wave + NW / 2) * WBUF + (k & 1) * Tile::FLOATS + lane;
+            const bool ends = i0 + 64 >= L1;   // the element's last row is one of these
             // FULL: every cell of the chunk lies inside the element, no validity masks
             auto steps = [&](auto full) {
             constexpr bool FULL = decltype(full)::value;
@@ -279,15 +294,14 @@ dtw_forward_kernel(const float* __restrict__ costs, const int* __restrict__ leng
                 const float z = (fast_exp2((m - diag) * c) + fast_exp2((m - up) * c)) +
                                 fast_exp2((m - cur) * c);
                 const float a = cv[u] + (m - tl * fast_log2(z));
-                const int col = t - lane;
-                const bool ok = FULL || ((unsigned)col < (unsigned)L2eff && in_band(ej, col + 1, bw));
+                const bool ok = FULL || (unsigned)(t - t_row) < (unsigned)cells;
                 cur = ok ? a : kPINF;
                 if (HELP) atile[u * 64] = cur;
                 else lane_store(outc + u * 64, ul4, cur);
                 pub[u] = cur;
                 // (the terminal cell never lies in a FULL chunk: lane 0's row is above
                 // L1 - 1, and the other lanes' columns stay below L2 - 1)
-                if (!FULL && ok && last_row && col == L2 - 1) terminal = cur;
+                if (!FULL && ends && ok && last_row && t - lane == L2 - 1) terminal = cur;
             }
             };
             if (bw < 0 && i0 + 63 < L1 && t0 >= 63 && t0 + P <= L2) steps(std::true_type{});
@@ -325,17 +339,43 @@ dtw_forward_kernel(const float* __restrict__ costs, const int* __restrict__ leng
         value[b] = NS > 0 ? terminal : ((L1 == 0 && L2 == 0) ? 0.0f : kPINF);
 }
 
+// Zeroes row[c0 .. c1), 16 bytes a lane where they are aligned.
+__device__ __forceinline__ void zero_span(float* row, int c0, int c1, int lane) {
+    if (c0 >= c1) return;
+    const int head = min(c0 + (int)((4 - (((uintptr_t)(row + c0) >> 2) & 3)) & 3), c1);
+    const int tail = head + ((c1 - head) & ~3);
+    if (c0 + lane < head) row[c0 + lane] = 0.0f;
+    for (int c = head + 4 * lane; c < tail; c += 256)
+        *reinterpret_cast<float4*>(row + c) = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+    if (tail + lane < c1) row[tail + lane] = 0.0f;
+}
+
+// Zeroes the marginals of a stripe's rows at the steps below a_end and from b_beg on,
+// which lie outside its band window.
+__device__ __forceinline__ void zero_off_band(float* pbase, int i0, int L1, int L2, int L2max,
+                                              int a_end, int b_beg, int lane) {
+    const int rows = min(64, L1 - i0);
+    for (int r = 0; r < rows; ++r) {
+        float* row = pbase + (size_t)(i0 + r) * L2max;
+        zero_span(row, 0, min(L2, a_end - r), lane);
+        zero_span(row, max(0, b_beg - r), L2, lane);
+    }
+}
+
 // The reverse sweep reads the forward's alpha table and nothing else: a cell's
 // softmin weights over its predecessors and its softmin value (the temperature
 // gradient's term) are both recomputed from the predecessors' alpha with the forward's
 // own arithmetic, so the costs are never loaded and the fused squared-Euclidean path
 // shares this sweep unchanged.
 //
-// HELP (unbanded parts of at most NW/2 stripes, e.g. 256-row elements): wave NW/2 + q
+// HELP (parts of at most NW/2 stripes, e.g. 256-row elements): wave NW/2 + q
 // helps the wave of stripe order q.  It loads the alpha rows one chunk ahead into that
 // wave's buffers (publishing hprog[q] = chunks loaded) and writes the chunk's marginals
 // out of a tile in its own, otherwise unused, buffers once wave q has finished the
-// chunk; wave q keeps only the row above and the boundary flows.
+// chunk; wave q keeps only the row above and the boundary flows.  With a band it also
+// zeroes the rows' cells off the band, which the sweeping wave would have its successors wait
+// for.  [16, 4096, 4096], bandwidth 64: 1.97 -> 1.53 ms; [512, 256, 256] without one 186 -> 170
+// us, from the interval of valid steps in the place of two tests per cell.
 template <int P, bool HELP = false>
 __global__ void __launch_bounds__(NW * 64)
 dtw_backward_kernel(const int* __restrict__ lengths,
@@ -413,7 +453,7 @@ dtw_backward_kernel(const int* __restrict__ lengths,
     }
 
     if constexpr (HELP) {
-        if (NL > NW / 2 || bandwidth >= 0) {   // never: the host picks HELP for these only
+        if (NL > NW / 2) {   // never: the host picks HELP for parts of at most NW/2
             if (threadIdx.x == 0) atomicOr(st, 2);
             return;
         }
@@ -421,31 +461,44 @@ dtw_backward_kernel(const int* __restrict__ lengths,
         if (q >= 0 && q < NL) {
             const int s = s_begin + NL - 1 - q;
             const int i0 = s * 64;
-            // unbanded: the window is every chunk and the table starts at step 0
+            // the stripe's window and its table, as the sweeping wave has them below
+            int t_lo, t_hi;
+            band_window(s, L1, L2, bw, t_lo, t_hi);
+            const bool none = t_lo > t_hi;
+            const int k_lo = __builtin_amdgcn_readfirstlane(none ? nch : (nsteps - 1 - t_hi) / P);
+            const int k_end =
+                __builtin_amdgcn_readfirstlane(none ? nch : (nsteps - 1 - t_lo) / P + 1);
+            const int sh = __builtin_amdgcn_readfirstlane(none ? 0 : t_lo / PF) * PF;
             const float* astripe = band_stripe(alpha_sk, b, elem_steps, s, stride);
             float* qbufs = smem + q * 2 * BUF;      // the sweeping wave's two chunk buffers
             float* obufs = smem + wave * 2 * BUF;   // its output tiles: this wave's buffers
             auto load = [&](int k) {
                 const int th = nsteps - 1 - k * P;
-                dma_rows<P, -1>(lds_address(qbufs + (k & 1) * BUF) + ABUF * 4, astripe, th - 2,
-                                ul4);
+                dma_rows<P, -1>(lds_address(qbufs + (k & 1) * BUF) + ABUF * 4, astripe,
+                                th - 2 - sh, ul4);
             };
             // whole row segments of marginals where rows start aligned (write_aligned):
             // P/4 stores per chunk instead of P
-            const bool aligned = (L2max & (P - 1)) == 0;
+            // (not with a band, whose window ends within segments)
+            const bool aligned = bw < 0.0f && (L2max & (P - 1)) == 0;
             AlignedCarry<P> carry;
             carry.clear();
-            if (nch > 0) {
-                load(0);
+            // the cells off the band: behind the sweep in the first quarter of the stripes,
+            // which come too early to wait for it, before it in the others
+            const bool behind = 4 * (NS - 1 - s) < NS;
+            const int a_end = nsteps - k_end * P, b_beg = nsteps - k_lo * P;
+            if (bw >= 0.0f && !behind) zero_off_band(pbase, i0, L1, L2, L2max, a_end, b_beg, lane);
+            if (k_lo < k_end) {
+                load(k_lo);
                 wait_vmcnt<0>();
-                publish(hprog, q, 1);
-                if (nch > 1) load(1);
+                publish(hprog, q, k_lo + 1);
+                if (k_lo + 1 < k_end) load(k_lo + 1);
             }
-            for (int k = 0; k < nch; ++k) {
-                if (k + 1 < nch) {
-                    // chunk k + 1's loads: the last issued at k = 0, else followed by the
+            for (int k = k_lo; k < k_end; ++k) {
+                if (k + 1 < k_end) {
+                    // chunk k + 1's loads: the last issued at k = k_lo, else followed by the
                     // marginal stores of chunk k - 1 (P, or P/4 aligned ones)
-                    if (k == 0) wait_vmcnt<0>();
+                    if (k == k_lo) wait_vmcnt<0>();
                     else if (aligned) wait_vmcnt<P / 4>();
                     else wait_vmcnt<P>();
                     publish(hprog, q, k + 2);   // also completes this wave's LDS reads
@@ -453,7 +506,7 @@ dtw_backward_kernel(const int* __restrict__ lengths,
                 // once wave q has finished chunk k, its buffer k & 1 takes chunk k + 2
                 // and its marginals (in output tile k & 1) leave
                 wait_for(prog, q, q * PROG_STRIDE + k + 1, st);
-                if (k + 2 < nch) load(k + 2);
+                if (k + 2 < k_end) load(k + 2);
                 if (aligned)
                     write_aligned<P, false>(obufs + (k & 1) * BUF, pbase, trash, carry, i0,
                                             L1max, L2max, lane, nsteps - 1 - k * P);
@@ -461,6 +514,7 @@ dtw_backward_kernel(const int* __restrict__ lengths,
                     write_tile<P, -1>(obufs + (k & 1) * BUF, pbase, trash, i0, L1, L2, L1max,
                                       L2max, lane, nsteps - 1 - k * P);
             }
+            if (bw >= 0.0f && behind) zero_off_band(pbase, i0, L1, L2, L2max, a_end, b_beg, lane);
         }
     }
 
@@ -469,8 +523,11 @@ dtw_backward_kernel(const int* __restrict__ lengths,
     for (int q = wave; q < NL; q += NW) {
         const int s = s_begin + NL - 1 - q;
         const int i0 = s * 64;
-        const int L2eff = (i0 + lane < L1) ? L2 : 0;
-        const float ej = band_centre(i0 + lane + 1, L1, L2);
+        // the row's valid cells, as in the forward
+        int t_row, cells;
+        band_columns(band_centre(i0 + lane + 1, L1, L2), bw, (i0 + lane < L1) ? L2 : 0, t_row,
+                     cells);
+        t_row += lane;
         // the terminal cell (L1, L2) starts with beta = 1
         const int term_step = (i0 + lane == L1 - 1) ? L2 - 1 + lane : -1000000;
         // the stripe's band window as reverse chunks [k_lo, k_end) (chunk k covers steps
@@ -520,18 +577,8 @@ dtw_backward_kernel(const int* __restrict__ lengths,
             }
         };
 
-        if (bw >= 0.0f) {
-            // cells of the stripe's rows at steps outside the window: off the band, zero
-            const int a_end = nsteps - k_end * P;   // steps below are not swept
-            const int b_beg = nsteps - k_lo * P;    // nor are steps from here on
-            const int rows = min(64, L1 - i0);
-            for (int r = 0; r < rows; ++r) {
-                float* row = pbase + (size_t)(i0 + r) * L2max;
-                const int c1 = min(L2, a_end - r);
-                for (int cc = lane; cc < c1; cc += 64) row[cc] = 0.0f;
-                for (int cc = max(0, b_beg - r) + lane; cc < L2; cc += 64) row[cc] = 0.0f;
-            }
-        }
+        if (!HELP && bw >= 0.0f)
+            zero_off_band(pbase, i0, L1, L2, L2max, nsteps - k_end * P, nsteps - k_lo * P, lane);
         publish(prog, wave, q * PROG_STRIDE + k_lo);   // nothing to do before the window
         if (k_lo == k_end) {
             publish(prog, wave, q * PROG_STRIDE + nch);
@@ -617,8 +664,7 @@ dtw_backward_kernel(const int* __restrict__ lengths,
 #pragma unroll
             for (int u = 0; u < P; ++u) {
                 const int t = t_hi - u;
-                const int col = t - lane;
-                const bool ok = FULL || ((unsigned)col < (unsigned)L2eff && in_band(ej, col + 1, bw));
+                const bool ok = FULL || (unsigned)(t - t_row) < (unsigned)cells;
                 const float a1 = A[u + 1];
                 const float bv_next = wave_shl1(bv);
                 const float upa = wave_shr1_or(a1, bv);
@@ -778,9 +824,9 @@ int launch_backward_p(const int* lengths, int B, int max_L1, int max_L2,
     const size_t lds = lds_backward_r(R, P);
     D2P_REQUIRE(lds <= kLdsLimit, "sequence too long for the LDS stripe rings");
     if (sp.G > 1) D2P_TRY(launch_flag_reset(ws.bflag, B * sp.G, st));
-    // helper waves for unbanded parts of at most NW/2 stripes (waves NW/2.. would idle)
+    // helper waves for parts of at most NW/2 stripes (waves NW/2.. would idle)
     const int part_stripes = sp.G > 1 ? sp.SPW : ns;
-    const bool help = bandwidth < 0 && part_stripes <= NW / 2 && dtw_helpers_enabled();
+    const bool help = part_stripes <= NW / 2 && dtw_helpers_enabled();
     auto kern = help ? dtw_backward_kernel<P, true> : dtw_backward_kernel<P, false>;
     D2P_HIP(hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize,
                                 (int)lds));
@@ -816,9 +862,9 @@ int launch_forward(const float* costs, const int* lengths, int B, int max_L1, in
     const size_t lds = lds_forward_r(R);
     D2P_REQUIRE(lds <= kLdsLimit, "sequence too long for the LDS stripe rings");
     if (sp.G > 1 && launch_split_reset(ws, B, sp.G, st) != D2P_OK) return D2P_ERR_HIP;
-    // helper waves for unbanded parts of at most NW/2 stripes (waves NW/2.. would idle)
+    // helper waves for parts of at most NW/2 stripes (waves NW/2.. would idle)
     const int part_stripes = sp.G > 1 ? sp.SPW : ns;
-    const bool help = bandwidth < 0 && part_stripes <= NW / 2 && dtw_helpers_enabled();
+    const bool help = part_stripes <= NW / 2 && dtw_helpers_enabled();
     auto kern = help ? dtw_forward_kernel<true> : dtw_forward_kernel<false>;
     D2P_HIP(hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize,
                                 (int)lds));

@@ -23,6 +23,24 @@ __device__ __forceinline__ bool in_band(float ej, int j, float bw) {
     return bw < 0.0f || fabsf((float)j - ej) <= bw;
 }
 
+// The columns [lo, lo + count) of a row that lie inside the element (of L2 columns) and
+// the band, by in_band() itself: |j - ej| is monotonic on either side of the centre also
+// after rounding, so they are an interval, whose ends lie within three columns of the
+// unrounded ones.  A sweep's per-cell test is then one subtraction and one comparison.
+__device__ __forceinline__ void band_columns(float ej, float bw, int L2, int& lo, int& count) {
+    int hi = L2 - 1;
+    lo = 0;
+    if (bw >= 0.0f) {
+        lo = max((int)floorf(fmaxf(ej - bw, -8.0f)) - 3, 0);
+        hi = min((int)ceilf(fminf(ej + bw, (float)L2 + 8.0f)) + 2, L2 - 1);
+        for (int i = 0; i < 8; ++i) {
+            if (!in_band(ej, lo + 1, bw)) ++lo;
+            if (!in_band(ej, hi + 1, bw)) --hi;
+        }
+    }
+    count = max(hi - lo + 1, 0);
+}
+
 // ------------------------------------------------------------ banded tables
 //
 // With a Sakoe-Chiba band every stripe sweeps only its window: the steps that can
