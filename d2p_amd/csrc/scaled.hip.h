@@ -16,11 +16,10 @@
 // marginal itself.  Sums are in 64 bits throughout: only E carries a 32-bit rounding.
 //
 // Range.  A lane's values may leave 2^-1022 .. 2^1023 of its chunk's scale only when
-// scores or costs move them by more than about 60 bits a step; such values become
-// infinite or NaN (or, for soft DTW, vanish), which the sweeps detect: they set
-// redo[b], and the log-domain sweeps recompute that element.  Values that vanish
-// against a finite neighbour (a gap costs at most kMaxGapBits, which the host checks)
-// contribute less than 2^-900 of it.
+// scores move them by more than about 60 bits a step; such values become infinite or NaN,
+// which the sweeps detect: they set redo[b], and the log-domain sweeps recompute that
+// element.  Values that vanish against a finite neighbour (a gap costs at most kMaxGapBits,
+// which the host checks) contribute less than 2^-900 of it.
 //
 // Pipeline.  Stripes of 64 rows, one wave each, a lane per row, one anti-diagonal per
 // step (wavefront.hip.h); at most 8 stripes per workgroup.  Longer elements, and
@@ -64,7 +63,7 @@ constexpr double kMaxGapBits = 40.0;
 // exponent of the SW scale: below it the restart term 1 would overflow
 constexpr int kMinExp = -900;
 
-enum Fam { SW, NW, AFF, NWAFF, DTW };
+enum Fam { SW, NW, AFF, NWAFF };
 
 template <Fam F>
 struct Traits {
@@ -76,7 +75,7 @@ struct Traits {
 };
 
 struct Consts {
-    float c;           // scores: log2(e)/T; costs: -log2(e)/T
+    float c;           // log2(e) / T
     double g, o, e;    // linear gap, open, extend factors
     double gc, oc, ec; // their base-2 exponents
 };
@@ -121,7 +120,7 @@ __host__ inline Mem carve(void* base, int B, int max_L1, int max_L2, int G) {
 }
 
 struct Args {
-    const float* m;       // scores or costs [B][L1max][L2max]
+    const float* m;       // scores [B][L1max][L2max]
     const int* lengths;   // [B][2] or null
     float* out;           // marginals
     float* value;
@@ -292,10 +291,6 @@ __device__ __forceinline__ void fwd_cell(const Consts& k, const FwdIn<F>& in, do
         t1 = F == SW ? __builtin_fma(in.f, d, in.one) : in.f * d;
         t3 = __builtin_fma(in.gf, u[0], k.g * v[0]);
         v[0] = __builtin_fma(E, t1, t3);
-    } else if constexpr (F == DTW) {
-        t1 = __builtin_fma(in.f, d + u[0], v[0]);
-        t3 = 0.0;
-        v[0] = E * t1;
     } else {
         // v = M, I, D; u[1] = the I state that the cell above feeds
         t1 = F == AFF ? __builtin_fma(in.f, d, in.one) : in.f * d;

@@ -125,6 +125,7 @@ __device__ __forceinline__ void export_boundary(const Ring<N>* ring, double* dst
 template <Fam F>
 __global__ void __launch_bounds__(MAXW * 64) fwd_kernel(const Args A) {
     using Tr = Traits<F>;
+    static_assert(Tr::AFFINE, "linear gaps: fwd2_sweep");
     extern __shared__ __align__(16) char smem[];
     __shared__ int prog[MAXW];
     __shared__ double zred[MAXW];
@@ -184,10 +185,10 @@ __global__ void __launch_bounds__(MAXW * 64) fwd_kernel(const Args A) {
         int K = 0;
 #pragma unroll
         for (int i = 0; i < Tr::NV; ++i) v[i] = 0.0;
-        if constexpr (F == NW || F == NWAFF) {       // column 0: a run of row + 1 gaps
+        if constexpr (F == NWAFF) {                  // column 0: a run of row + 1 gaps
             const double e = edge_log2<F>(A.k, i0 + lane + 1);
             K = (int)floor(e);
-            v[F == NW ? 0 : 1] = exp2(e - (double)K);
+            v[1] = exp2(e - (double)K);
         }
         fwd_pass<F>(A.k, v, p);
 
@@ -238,15 +239,15 @@ __global__ void __launch_bounds__(MAXW * 64) fwd_kernel(const Args A) {
                                            rin->k[min(3, nch - 1) & (RCH - 1)]);
 #pragma unroll
                 for (int i = 0; i < Tr::NP; ++i) ring[i][0] = scale2(ring[i][0], ka - kr);
-            } else if (F == NW || F == NWAFF) {      // row 0: a run of j gaps
+            } else if (F == NWAFF) {                 // row 0: a run of j gaps
                 const double e = edge_log2<F>(A.k, k * P + 1);
                 kr = (int)floor(e);
                 double x = exp2(e - (double)kr);
 #pragma unroll
                 for (int j = 0; j < P; ++j) {
                     ring[0][j] = x;
-                    if (F == NWAFF) ring[Tr::NP - 1][j] = A.k.o * x;
-                    x *= F == NW ? A.k.g : A.k.e;
+                    ring[Tr::NP - 1][j] = A.k.o * x;
+                    x *= A.k.e;
                 }
             } else {
 #pragma unroll
@@ -270,32 +271,25 @@ __global__ void __launch_bounds__(MAXW * 64) fwd_kernel(const Args A) {
             // (infinities and NaN stay: they are looked for after the last chunk)
             int Kn = K + (ex > -1023 && ex < 1024 ? ex : 0);
             if (Tr::LOCAL) Kn = max(Kn, kMinExp);
-            if (F == SW || F == AFF || F == DTW) {
+            if (Tr::LOCAL) {
                 const int started = k * P;           // lanes below have started
                 if (started < 64) {
                     const int kb = k == 0 ? kr : __builtin_amdgcn_readlane(Kn, started - 1);
                     if (lane >= started) Kn = kb;
                 }
             }
-            if constexpr (F == DTW) {
-                // a started lane whose value has vanished: out of the 64-bit range
-                if (__builtin_amdgcn_ballot_w64(lane_ok && lane < k * P && k * P - lane <= L2 &&
-                                                ex < -900) != 0 && lane == 0)
-                    flag_redo(A.redo + b);
-            }
             // lane 0's diagonal input at its first cell: the cell above column 0 (other lanes
             // have it from the lane above)
             if (k == 0) {
                 kr_prev = kr;
-                if (F == DTW) d = i0 == 0 ? 1.0 : 0.0;
-                if constexpr (F == NW || F == NWAFF) {
+                if constexpr (F == NWAFF) {
                     const double e = i0 > 0 ? edge_log2<F>(A.k, i0) : 0.0;
                     const int ke = (int)floor(e);
                     d = scale2(exp2(e - (double)ke), ke - kr);
                 }
             }
             // (zeros from above the first stripe: any finite factor will do)
-            if (!ring_in && !(F == NW || F == NWAFF)) kr = __builtin_amdgcn_readlane(Kn, 0);
+            if (!ring_in && F == AFF) kr = __builtin_amdgcn_readlane(Kn, 0);
             const int delta = K - Kn;
 #pragma unroll
             for (int i = 0; i < Tr::NV; ++i) v[i] = scale2(v[i], delta);
@@ -506,8 +500,8 @@ __device__ __forceinline__ void store_segments(const OutTile* o, float* obase, f
 // ------------------------------------------------------------------ results
 
 // Value and parameter gradients of element b from the sums r: linear gaps {gaps (global:
-// matches), -, sum P s}, affine {opens, extends (global: matches), sum P s}, soft DTW
-// {-, -, sum P c}; S = T log Z.  A global path of M matches has L1 + L2 - 2 M gaps.
+// matches), -, sum P s}, affine {opens, extends (global: matches), sum P s}; S = T log Z.
+// A global path of M matches has L1 + L2 - 2 M gaps.
 template <Fam F>
 __device__ inline void finalize(const Args& A, int b, int L1, int L2, const double* r, double S) {
     const bool empty = L1 <= 0 || L2 <= 0;
@@ -524,15 +518,13 @@ __device__ inline void finalize(const Args& A, int b, int L1, int L2, const doub
         path += g0 * A.gap + g1 * A.ext;
     } else if constexpr (F == SW) {
         path += g0 * A.gap;
-    } else if constexpr (F == AFF) {
-        path += g0 * A.gap + g1 * A.ext;
     } else {
-        value = empty ? (L1 == L2 ? 0.0 : (double)kPINF) : -S;
+        path += g0 * A.gap + g1 * A.ext;
     }
     A.value[b] = (float)value;
     if (A.grad0) A.grad0[b] = (float)g0;
     if (A.grad1) A.grad1[b] = (float)g1;
-    A.gradT[b] = F == DTW && empty ? 0.0f : (float)((value - path) / A.T);
+    A.gradT[b] = (float)((value - path) / A.T);
 }
 
 // The element's partition, as mantissa in [1, 2) and exponent (zm = 0: out of range).
@@ -672,7 +664,7 @@ __global__ void __launch_bounds__((Traits<F>::AFFINE ? 4 : MAXW) * 64) bwd_kerne
 
         // own state: y = E b (of M, affine) and its previous step's yo; bb = b (bI, affine);
         // bd = bD.  Passed up: w, what the row above takes from this column and the next,
-        //   linear gap  y[j+1] + g b[j];  soft DTW  y[j+1] + y[j];  affine  y[j+1] (and bI[j])
+        //   linear gap  y[j+1] + g b[j];  affine  y[j+1] (and bI[j])
         double y = 0.0, bb = 0.0, bd = 0.0, w = 0.0;
         int K = 0;
 
@@ -759,13 +751,7 @@ __global__ void __launch_bounds__((Traits<F>::AFFINE ? 4 : MAXW) * 64) bwd_kerne
                 if (ring_in) kr = __builtin_amdgcn_readfirstlane(rin->k[max(kf - 4, 0) & (RCH - 1)]);
             }
             {
-                const int ex = exponent(F == DTW ? y : bb);
-                if constexpr (F == DTW) {
-                    if (__builtin_amdgcn_ballot_w64(lane_ok && lane >= first &&
-                                                    (kf + 1) * P - lane >= 0 && ex < -900) != 0 &&
-                        lane == 0)
-                        flag_redo(A.redo + b);
-                }
+                const int ex = exponent(bb);
                 int Kn = K + (ex > -1023 && ex < 1024 ? ex : 0);
                 if (first > 0 || rows < 64) {
                     const int kb = first < rows ? __builtin_amdgcn_readlane(Kn, min(first, 63)) : kr;
@@ -776,7 +762,7 @@ __global__ void __launch_bounds__((Traits<F>::AFFINE ? 4 : MAXW) * 64) bwd_kerne
                 const int delta = K - Kn;
                 y = scale2(y, delta);
                 w = scale2(w, delta);
-                if (F != DTW) bb = scale2(bb, delta);
+                bb = scale2(bb, delta);
                 if (Tr::AFFINE) bd = scale2(bd, delta);
                 K = Kn;
             }
@@ -791,8 +777,7 @@ __global__ void __launch_bounds__((Traits<F>::AFFINE ? 4 : MAXW) * 64) bwd_kerne
                 const int su = shr1(sum, 0) - zk;
                 if (lane > 0) d = scale2(d * invZ, su);
                 const int Kb_up = shr1(K, 0);
-                // (zeros come from above the first stripe, but for soft DTW's cell (0, 0))
-                const bool top = above || GLOBAL || (F == DTW && kf == 0);
+                const bool top = above || GLOBAL;     // (else zeros come from above)
                 in.f = lane > 0 ? scale2(1.0, K - Kb_up)
                                 : (top ? scale2(invZ, ka4 + K - zk) : 0.0);
                 in.gf = A.k.g * in.f;
@@ -900,14 +885,6 @@ __global__ void __launch_bounds__((Traits<F>::AFFINE ? 4 : MAXW) * 64) bwd_kerne
                         else gacc = __builtin_fma(FULL || ok ? t3[j] : 0.0, bn, gacc);
                         w = __builtin_fma(A.k.g, bn, y);
                         bb = bn;
-                    } else if constexpr (F == DTW) {
-                        double bn = __builtin_fma(fb, wd, y);
-                        if (end) bn = scale2(1.0, -K);
-                        yn = E[j] * bn;
-                        if (!FULL) yn = ok ? yn : 0.0;
-                        Pm = t1[j] * yn;
-                        if (!FULL) Pm = ok ? Pm : 0.0;
-                        w = y + yn;
                     } else {
                         const double bi = shl1(bb, fl[z][Tr::NQ - 1][e]);      // bI of (i+1, j)
                         const double w0 = F == AFF ? __builtin_fma(fb, wd, one) : fb * wd;
@@ -1016,7 +993,7 @@ __global__ void __launch_bounds__((Traits<F>::AFFINE ? 4 : MAXW) * 64) bwd_kerne
 
 // ------------------------------------------------------------------ two waves a stripe
 
-// Families with one state (soft SW and NW with linear gaps, soft DTW) run two waves per
+// Families with one state (linear gaps) run two waves per
 // stripe: a sweeping wave that carries the recurrence and nothing else, and a helper on
 // the same SIMD that does what does not depend on it (loads, exponentials, the last row
 // and, in the reverse sweep, the recomputation and the marginals).  A lone wave issues
@@ -1157,17 +1134,10 @@ __device__ __forceinline__ void fwd2_sweep(const Args& A, int b, int part) {
                 const int kb = k == 0 ? kr : __builtin_amdgcn_readlane(Kn, max(k * P - 1, 0));
                 if (lane >= k * P) Kn = kb;
             }
-            if constexpr (F == DTW) {
-                // a started lane whose value has vanished: out of the 64-bit range
-                if (__builtin_amdgcn_ballot_w64(lane_ok && lane < k * P && k * P - lane <= L2 &&
-                                                ex < -900) != 0 && lane == 0)
-                    flag_redo(A.redo + b);
-            }
             // lane 0's diagonal input at its first cell: the cell above column 0 (other lanes
             // have it from the lane above)
             if (k == 0) {
                 kr_prev = kr;
-                if (F == DTW) d = i0 == 0 ? 1.0 : 0.0;
                 if constexpr (F == NW) {
                     const double e = i0 > 0 ? edge_log2<F>(A.k, i0) : 0.0;
                     const int ke = (int)floor(e);
@@ -1450,7 +1420,7 @@ __device__ __forceinline__ void bwd2_sweep(const Args& A, int b, int part) {
             for (int i = lane; i < RING; i += 64) rings[wave + 1].v[0][i] = 0.0;
         }
         // y = E b of the last cell and b; w: what the row above takes from a column and
-        // the next, y[j+1] + g b[j] (soft DTW: y[j+1] + y[j])
+        // the next, y[j+1] + g b[j]
         double y = 0.0, bb = 0.0, w = 0.0;
         int K = 0, kr = 0;
         int pp = -1, pc = -1, ph = -1, pu = -1;
@@ -1485,13 +1455,7 @@ __device__ __forceinline__ void bwd2_sweep(const Args& A, int b, int part) {
             // the chunk's scale, as in the forward: lanes not started take that of the lowest
             // started one (or the ring's), lanes past the element's rows that of the last row
             const int first = max((kf + 1) * P - L2 + 1, 0);    // lowest started lane
-            const int ex = exponent(F == DTW ? y : bb);
-            if constexpr (F == DTW) {
-                if (__builtin_amdgcn_ballot_w64(lane_ok && lane >= first &&
-                                                (kf + 1) * P - lane >= 0 && ex < -900) != 0 &&
-                    lane == 0)
-                    flag_redo(A.redo + b);
-            }
+            const int ex = exponent(bb);
             int Kn = K + (ex > -1023 && ex < 1024 ? ex : 0);
             if (first > 0 || rows < 64) {
                 const int kb = first < rows ? __builtin_amdgcn_readlane(Kn, min(first, 63)) : kr;
@@ -1503,7 +1467,7 @@ __device__ __forceinline__ void bwd2_sweep(const Args& A, int b, int part) {
                 const int delta = K - Kn;
                 y = scale2(y, delta);
                 w = scale2(w, delta);
-                if (F != DTW) bb = scale2(bb, delta);
+                bb = scale2(bb, delta);
                 K = Kn;
             }
             if (!ring_in) kr = __builtin_amdgcn_readlane(K, 63);   // (zeros from below)
@@ -1543,12 +1507,9 @@ __device__ __forceinline__ void bwd2_sweep(const Args& A, int b, int part) {
                     if (!FULL && F == NW && owns_end && t0 + j == t_end && lane == lane_end)
                         bn = scale2(1.0, -K);
                     bn = __builtin_fma(fb, wd, bn);
-                    if (!FULL && F == DTW && owns_end && t0 + j == t_end && lane == lane_end)
-                        bn = scale2(1.0, -K);
                     if (!FULL) bn = ok ? bn : 0.0;
                     const double yn = (double)(FULL || ok ? E[j] : 0.0f) * bn;
-                    if (F == DTW) w = y + yn;
-                    else w = __builtin_fma(A.k.g, bn, y);
+                    w = __builtin_fma(A.k.g, bn, y);
                     bb = bn;
                     y = yn;
                     wh[j & 3] = w;
@@ -1626,7 +1587,7 @@ __device__ __forceinline__ void bwd2_sweep(const Args& A, int b, int part) {
                 if (lane > 0) d = scale2(d * invZ, su);
                 const int K_up = shr1(K, 0);         // (not inside the select: every lane active)
                 in.f = lane > 0 ? scale2(1.0, K - K_up) : scale2(invZ, ka4 + K - zk);
-                if (F != NW && !above && !(F == DTW && kf == 0) && lane == 0) in.f = 0.0;
+                if (F != NW && !above && lane == 0) in.f = 0.0;
                 in.gf = A.k.g * in.f;
                 in.one = Tr::LOCAL ? scale2(invZ, K - zk) : 0.0;
             }
@@ -1663,7 +1624,7 @@ __device__ __forceinline__ void bwd2_sweep(const Args& A, int b, int part) {
                         v = ok ? vn : (F == NW ? v : 0.0);
                         d = u;
                         const double bs = b4[z][e];
-                        const double Pm = (F == DTW ? v : v - t3) * bs;
+                        const double Pm = (v - t3) * bs;
                         if (F == SW) gacc = __builtin_fma(t3, bs, gacc);
                         if (F == NW) gacc += Pm;
                         (bq + j * BROW)[lane] = (float)Pm;
@@ -1845,10 +1806,10 @@ inline Split choose_parts(int B, int ns) {
     return sp;
 }
 
-inline Consts consts(Fam f, double T, double gap_or_open, double ext) {
+inline Consts consts(double T, double gap_or_open, double ext) {
     Consts k;
     const double c = 1.4426950408889634074 / T;
-    k.c = (float)(f == DTW ? -c : c);
+    k.c = (float)c;
     k.gc = k.oc = gap_or_open * c;
     k.ec = ext * c;
     k.g = k.o = exp2(k.gc);

@@ -31,7 +31,7 @@ int run_scaled(const float* scores, const int* lengths, int B, int max_L1, int m
     A.B = B;
     A.L1max = max_L1;
     A.L2max = max_L2;
-    A.k = sc::consts(global ? sc::NW : sc::SW, T, gap, 0.0);
+    A.k = sc::consts(T, gap, 0.0);
     const size_t room = (size_t)((char*)ws.brow - (char*)ws.alpha_sk);
     if (global) return sc::run<sc::NW>(A, ws.alpha_sk, room, done, st, "nw_forward", "nw_backward");
     return sc::run<sc::SW>(A, ws.alpha_sk, room, done, st, "sw_forward", "sw_backward");

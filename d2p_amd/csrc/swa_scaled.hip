@@ -34,7 +34,7 @@ int run_scaled(const float* scores, const int* lengths, int B, int max_L1, int m
     A.B = B;
     A.L1max = max_L1;
     A.L2max = max_L2;
-    A.k = sc::consts(nwa ? sc::NWAFF : sc::AFF, T, go, ge);
+    A.k = sc::consts(T, go, ge);
     const size_t room = (size_t)((char*)ws.brow - (char*)ws.alpha_sk);
     if (nwa)
         return sc::run<sc::NWAFF>(A, ws.alpha_sk, room, done, st, "nwa_forward", "nwa_backward");
