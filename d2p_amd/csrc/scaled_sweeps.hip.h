@@ -200,7 +200,9 @@ __global__ void __launch_bounds__(MAXW * 64) fwd_kernel(const Args A) {
         };
 #pragma unroll
         for (int k = 0; k < NT; ++k) load(k);
-        wait_vmcnt<4 * (NT - 1)>();
+        // (all of them: the waits below count the loads and stores of three chunks, which the
+        // first chunks do not have behind them)
+        wait_vmcnt<0>();
         float sN[P];
         read_quads<P, 1>(tile, lane, sN);
         double bw[Tr::NP];       // last row of the previous chunk, on its way to memory

@@ -113,3 +113,20 @@ def test_elements_out_of_range(cuda, L1, L2, op, gaps):
     assert err[1] <= math.sqrt(L1 + L2) * 2.0 ** -15, err
     v = got[0].cpu().numpy().astype(np.float64)
     assert np.all(np.abs(v - want[0]) <= 1e-5 * np.abs(want[0]) + 1e-5), (v, want[0])
+
+
+@pytest.mark.parametrize("B,L1,L2", [(300, 130, 66), (40, 300, 200)])
+def test_affine_calls_repeat_bit_for_bit(cuda, B, L1, L2):
+    # a wave reads its first chunks' scores only once they have arrived: workgroups that
+    # start on LDS with other contents (a NaN element's, say) give the same results
+    s, _ = _inputs(B, L1, L2, False)
+    x = torch.from_numpy(s).to(cuda)
+    want = d2p_amd.soft_sw_affine_with_grads(x, -2.0, -0.5, 1.0, None)
+    y = x.clone()
+    y[1, 3, 4] = float("nan")
+    for _ in range(5):
+        got = d2p_amd.soft_sw_affine_with_grads(y, -2.0, -0.5, 1.0, None)
+        torch.cuda.empty_cache()
+        keep = [i for i in range(B) if i != 1]
+        for a, b in zip(want, got):
+            assert torch.equal(a[keep], b[keep])
