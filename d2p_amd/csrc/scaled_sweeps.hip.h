@@ -1,6 +1,7 @@
 // scaled_sweeps.hip.h -- the forward and reverse sweep kernels of scaled.hip.h and
 // their launches, one instantiation per family.
 #pragma once
+#include <float.h>
 #include <limits.h>
 #include <stdlib.h>
 
@@ -1319,7 +1320,8 @@ __global__ void __launch_bounds__(MAXW2 * 64) fwd2_kernel(const Args A) {
 
 // The end of a chunk of the reverse sweep: its marginals, which lie by step and lane in
 // the rows of the b buffer, to memory, and the sum of P log2 E over the lane's cells
-// (log2 E = c s; no marginal where E is 0).  Row r = 16 i + r0 completes its segment of
+// (log2 E = c s, over the whole range of E: there is no marginal where it is 0, and where it is
+// infinite the element is out of range).  Row r = 16 i + r0 completes its segment of
 // columns 16 (kf - i) .. + 15: column 4 p + e of it was made in step n = 4 p + e + r0 of this
 // chunk or, from 16 on, in step n - 16 of the chunk before, whose share is kept in cy.
 // The buffer is free once everything has been read.
@@ -1349,7 +1351,7 @@ __device__ __forceinline__ double emit_chunk(float* bq, const float* tq, f32x4 (
 #pragma unroll
         for (int e = 0; e < 4; ++e)
             ps = fmaf((bq + (4 * g + e) * BROW)[l],
-                      fast_log2(__builtin_amdgcn_fmed3f(E4[e], 1e-37f, 1e37f)), ps);
+                      fast_log2(__builtin_amdgcn_fmed3f(E4[e], FLT_MIN, FLT_MAX)), ps);
     }
     __asm__ volatile("" : "+v"(ps)::"memory");
     post(prog, word, done);

@@ -53,6 +53,27 @@ def _tol(s, m, T):
     return 8.0 * math.sqrt(m) * delta
 
 
+def _check(got, want, s, gaps, T, tol, glob=False):
+    """Every output of the elements against the 64-bit oracle's.  tol bounds the logarithm of
+    a marginal, so a sum of marginals is off by at most tol times its terms' sizes: the
+    gaps are counted by such a sum (global alignment: by L1 + L2 less two for each match),
+    and dS/dT = (S - sum P s - sum gaps n_gap) / T has the terms that `terms` adds up.  What is
+    rounded to 32 bits at the end adds 2^-23 of itself."""
+    got = [x.cpu().numpy().astype(np.float64) for x in got]
+    value, post = want[0], want[1]
+    assert np.all(np.abs(got[0] - value) <= T * tol + 2.0 ** -23 * np.abs(value)), (got[0], value)
+    err = np.abs(got[1] - post).max()
+    assert err <= tol, (err, tol)
+    matches = post.sum(axis=(1, 2))
+    terms = np.abs(value) + (post * np.abs(np.where(post > 0, s, 0))).sum(axis=(1, 2))
+    for n, (gap, g, w) in enumerate(zip(gaps, got[2:-1], want[2:-1])):
+        bound = tol * (np.abs(w) + (4 * matches + 1 if glob else 0)) + 2.0 ** -22 * np.abs(w)
+        assert np.all(np.abs(g - w) <= bound + 1e-30), (n, g, w, bound)
+        terms = terms + np.abs(gap) * (np.abs(w) + (4 * matches if glob else 0))
+    bound = (tol + 2.0 ** -22) * terms / T
+    assert np.all(np.abs(got[-1] - want[-1]) <= bound), (got[-1], want[-1], bound)
+
+
 @pytest.mark.parametrize("nw", [False, True])
 @pytest.mark.parametrize("B,L1,L2,T,gap,parts,ragged", CASES)
 def test_scaled_sweeps_match_double_oracle(cuda, monkeypatch, B, L1, L2, T, gap, parts, ragged,
@@ -62,16 +83,12 @@ def test_scaled_sweeps_match_double_oracle(cuda, monkeypatch, B, L1, L2, T, gap,
     s, lengths = _inputs(B, L1, L2, ragged)
     op = "soft_nw" if nw else "soft_sw"
     lt = None if lengths is None else torch.from_numpy(lengths).to(cuda)
-    got = getattr(d2p_amd, op)(torch.from_numpy(s).to(cuda), gap, T, lengths=lt)
+    got = getattr(d2p_amd, op + "_with_grads")(torch.from_numpy(s).to(cuda), gap, T, lt)
     n = min(B, 9)
     idx = list(range(n - 1)) + [B - 1]
     want = getattr(O.get("oracle64"), op)(s[idx].astype(np.float64), gap, T,
                                            None if lengths is None else lengths[idx])
-    tol = _tol(s, min(L1, L2), T)
-    value = got[0].cpu().numpy()[idx].astype(np.float64)
-    assert np.all(np.abs(value - want[0]) <= T * tol + 2.0 ** -23 * np.abs(want[0])), value
-    err = np.abs(got[1].cpu().numpy()[idx] - want[1]).max()
-    assert err <= tol, (err, tol)
+    _check([x[idx] for x in got], want, s[idx], (gap,), T, _tol(s, min(L1, L2), T), nw)
 
 
 @pytest.mark.parametrize("nw", [False, True])
@@ -83,16 +100,14 @@ def test_scaled_affine_sweeps_match_double_oracle(cuda, monkeypatch, B, L1, L2, 
     s, lengths = _inputs(B, L1, L2, ragged)
     op = "soft_nw_affine" if nw else "soft_sw_affine"
     lt = None if lengths is None else torch.from_numpy(lengths).to(cuda)
-    got = getattr(d2p_amd, op)(torch.from_numpy(s).to(cuda), gap - 1.0, gap / 2, T, lengths=lt)
+    got = getattr(d2p_amd, op + "_with_grads")(torch.from_numpy(s).to(cuda), gap - 1.0, gap / 2,
+                                               T, lt)
     n = min(B, 9)
     idx = list(range(n - 1)) + [B - 1]
     want = getattr(O.get("oracle64"), op)(s[idx].astype(np.float64), gap - 1.0, gap / 2, T,
                                           None if lengths is None else lengths[idx])
-    tol = _tol(s, min(L1, L2), T)
-    value = got[0].cpu().numpy()[idx].astype(np.float64)
-    assert np.all(np.abs(value - want[0]) <= T * tol + 2.0 ** -23 * np.abs(want[0])), value
-    err = np.abs(got[1].cpu().numpy()[idx] - want[1]).max()
-    assert err <= tol, (err, tol)
+    _check([x[idx] for x in got], want, s[idx], (gap - 1.0, gap / 2), T,
+           _tol(s, min(L1, L2), T), nw)
 
 
 @pytest.mark.parametrize("op,gaps", [("soft_sw", (-1.0,)), ("soft_nw", (-1.0,)),
@@ -130,3 +145,20 @@ def test_affine_calls_repeat_bit_for_bit(cuda, B, L1, L2):
         keep = [i for i in range(B) if i != 1]
         for a, b in zip(want, got):
             assert torch.equal(a[keep], b[keep])
+
+
+@pytest.mark.parametrize("op", ["soft_sw", "soft_nw"])
+@pytest.mark.parametrize("T", [0.2, 1.0])
+@pytest.mark.parametrize("B,L1,L2", [(4, 100, 120),     # both sweeps in one launch
+                                     (4, 257, 130),     # two parts
+                                     (300, 100, 45)])   # one reverse wave a stripe
+def test_strong_scores(cuda, B, L1, L2, T, op):
+    # one cell each whose factor lies at the upper end of the 32-bit range, 2^121 to 2^127
+    # (whose rounding, 2^-24 of 127 bits, adds to that of the ordinary ones on its path)
+    s, _ = _inputs(B, L1, L2, False)
+    tol = math.hypot(_tol(s, min(L1, L2), T), 8.0 * 2.0 ** -24 * 127.0)
+    for b, x in enumerate((84.0, 86.0, 88.0)):
+        s[b, L1 // 2, L2 // 2] = x * T
+    got = getattr(d2p_amd, op + "_with_grads")(torch.from_numpy(s).to(cuda), -1.0, T, None)
+    want = getattr(O.get("oracle64"), op)(s[:4].astype(np.float64), -1.0, T, None)
+    _check([x[:4] for x in got], want, s[:4], (-1.0,), T, tol, op == "soft_nw")
