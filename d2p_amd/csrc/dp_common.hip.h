@@ -64,6 +64,13 @@ __device__ __forceinline__ float max4_raw(float a, float b, float c, float d) {
     return m;
 }
 
+// min(a, b, c) as one v_min3_f32, for the same reason.
+__device__ __forceinline__ float min3_raw(float a, float b, float c) {
+    float m;
+    __asm__("v_min3_f32 %0, %1, %2, %3" : "=v"(m) : "v"(a), "v"(b), "v"(c));
+    return m;
+}
+
 __device__ __forceinline__ float lane_bcast(float v, int lane) {
     return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), lane));
 }

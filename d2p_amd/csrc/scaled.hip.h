@@ -15,11 +15,16 @@
 // rebuilds the chunk's values from it in registers, in the scale that makes a b / Z the
 // marginal itself.  Sums are in 64 bits throughout: only E carries a 32-bit rounding.
 //
-// Range.  A lane's values may leave 2^-1022 .. 2^1023 of its chunk's scale only when
-// scores move them by more than about 60 bits a step; such values become infinite or NaN,
-// which the sweeps detect: they set redo[b], and the log-domain sweeps recompute that
-// element.  Values that vanish against a finite neighbour (a gap costs at most kMaxGapBits,
-// which the host checks) contribute less than 2^-900 of it.
+// Range.  Scores that move a lane's values up by more than about 60 bits a step take them
+// beyond 2^1023 of its chunk's scale: they become infinite or NaN, which the sweeps detect.
+// They set redo[b], and the log-domain sweeps recompute that element.
+// Downwards nothing becomes infinite.  E is 0 below 2^-149 (and rounded below 2^-126), and
+// values below 2^-1022 of the scale are lost.  Where two gaps go round any match (linear
+// gaps, and global affine ones, whose gaps follow each other in either order) they bound both:
+// a gap costs at most kMaxGapBits, which the host checks, so what is left out weighs less than
+// 2^(80 - 126) of what goes round it.  Local affine alignment has to match through the cell: the
+// forward keeps the largest factor below 2^-126 that it met, and element_partition() says
+// whether it can be left out (a mask: yes) or the element is out of range.
 //
 // Pipeline.  Stripes of 64 rows, one wave each, a lane per row, one anti-diagonal per
 // step (wavefront.hip.h); at most 8 stripes per workgroup.  Longer elements, and
@@ -60,6 +65,12 @@ constexpr int LEAD = 5;             // chunks a stripe runs behind its producer
 constexpr int MAXW = 8;             // waves per workgroup
 constexpr int MAXS_SPLIT = 6;       // stripes per part beside the two copying waves
 constexpr double kMaxGapBits = 40.0;
+// log2 of the least factor E that 32 bits hold in full
+constexpr float kMinBits = -126.0f;
+// local affine elements with smaller factors (element_partition): log2 of Z at most, and log2 of
+// the share of Z of the paths through one such cell at most (2^20 cells: 2^-40 in all)
+constexpr int kMaxMaskedExp = 850;
+constexpr double kNoShare = -60.0;
 // exponent of the SW scale: below it the restart term 1 would overflow
 constexpr int kMinExp = -900;
 
@@ -92,7 +103,7 @@ struct Mem {
     int* kexp;      // [B][part][nch] forward boundary exponents (split)
     double* flow;   // [B][part][plane NQ][16 nch] reverse flows by step (split)
     int* kflow;     // [B][part][nch] their exponents
-    double* zpart;  // [B][part][2] partition (mantissa, exponent)
+    double* zpart;  // [B][part][3] partition (mantissa, exponent), log2 of the largest E left out
     size_t bytes;
 };
 
@@ -114,7 +125,7 @@ __host__ inline Mem carve(void* base, int B, int max_L1, int max_L2, int G) {
     m.kexp = (int*)take(pt * nch * 4);
     m.flow = (double*)take(pt * Tr::NQ * P * nch * 8);
     m.kflow = (int*)take(pt * nch * 4);
-    m.zpart = (double*)take(pt * 2 * 8);
+    m.zpart = (double*)take(pt * 3 * 8);
     m.bytes = (size_t)(p - (char*)base);
     return m;
 }

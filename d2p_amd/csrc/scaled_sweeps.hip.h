@@ -131,6 +131,7 @@ __global__ void __launch_bounds__(MAXW * 64) fwd_kernel(const Args A) {
     __shared__ int prog[MAXW];
     __shared__ double zred[MAXW];
     __shared__ int kred[MAXW];
+    __shared__ float lred[MAXW];
     int b, part;
     split_decode(blockIdx.x, A.G, b, part);
     if (b >= A.B) return;
@@ -161,6 +162,7 @@ __global__ void __launch_bounds__(MAXW * 64) fwd_kernel(const Args A) {
 
     double zsum = 0.0;      // this wave's share of the partition, scaled by 2^-zk
     int zk = -(1 << 28);
+    float low = -FLT_MAX;   // log2 of the largest factor below kMinBits
     if (wave < n) {
         const int s = s0 + wave, i0 = 64 * s;
         const int rows = min(64, L1 - i0);
@@ -261,6 +263,20 @@ __global__ void __launch_bounds__(MAXW * 64) fwd_kernel(const Args A) {
             double Ed[P];
 #pragma unroll
             for (int i = 0; i < P; ++i) Ed[i] = (double)fast_exp2(sN[i] * A.k.c);
+            if constexpr (F == AFF) {
+                float least = min3_raw(sN[0], sN[1], sN[2]);
+#pragma unroll
+                for (int i = 3; i < P - 1; i += 2) least = min3_raw(least, sN[i], sN[i + 1]);
+                least = min3_raw(least, sN[P - 1], sN[P - 1]);
+                if (__builtin_amdgcn_ballot_w64(least * A.k.c < kMinBits) != 0) {
+#pragma unroll
+                    for (int i = 0; i < P; ++i) {
+                        const float x = sN[i] * A.k.c;
+                        if (lane_ok && (unsigned)(k * P + i - lane) < (unsigned)L2 && x < kMinBits)
+                            low = fmaxf(low, fmaxf(x, -1e30f));
+                    }
+                }
+            }
             // next chunk's scores: its loads were issued three chunks ago, and at least two
             // stores and, in each of the two chunks since, four loads and two stores follow
             wait_vmcnt<2 + 6 * (NT - 2)>();
@@ -415,6 +431,10 @@ __global__ void __launch_bounds__(MAXW * 64) fwd_kernel(const Args A) {
             zred[wave] = zsum;
             kred[wave] = km;
         }
+        if constexpr (F == AFF) {
+            low = wave_reduce(low, [](float a, float b) { return fmaxf(a, b); });
+            if (lane == 0) lred[wave] = low;
+        }
     }
     __syncthreads();
     if (threadIdx.x == 0) {
@@ -431,9 +451,14 @@ __global__ void __launch_bounds__(MAXW * 64) fwd_kernel(const Args A) {
             z = scale2(z, max(kz - km, -4000)) + scale2(zred[w], max(kred[w] - km, -4000));
             kz = km;
         }
-        double* zp = A.mem.zpart + ((size_t)b * A.G + part) * 2;
+        double* zp = A.mem.zpart + ((size_t)b * A.G + part) * 3;
         zp[0] = z;
         zp[1] = (double)kz;
+        if constexpr (F == AFF) {
+            float least = -FLT_MAX;
+            for (int w = 0; w < n; ++w) least = fmaxf(least, lred[w]);
+            zp[2] = (double)least;
+        }
     }
 }
 
@@ -531,13 +556,26 @@ __device__ inline void finalize(const Args& A, int b, int L1, int L2, const doub
 }
 
 // The element's partition, as mantissa in [1, 2) and exponent (zm = 0: out of range).
+//
+// Local affine gaps: a step from one kind of gap to the other has to match in between, so
+// no detour of two gaps bounds what a factor below 2^kMinBits, which is not kept, would
+// weigh.  Such a factor E may be left out if
+//  * E Z is small: a path through its cell is an alignment before it and one behind it (and
+//    gaps, of at most 1 each), of at most Z each, so its share of Z is at most E Z;
+//  * 2^-K, the restart term in the lanes' scale, is within the 64-bit range with room for
+//    another factor (K is at most the exponent of Z, and of Z times the rows in the reverse
+//    sweep): beside a cell without weight nothing else keeps a row from its neighbour's
+//    scale.  What is lost below 2^-1022 of the scale is then nothing beside a restart.
+template <Fam F>
 __device__ __forceinline__ void element_partition(const Args& A, int b, double& zm, int& zk) {
     zm = 0.0;
     zk = -(1 << 28);
+    double low = -FLT_MAX;
     for (int g = 0; g < A.G; ++g) {
-        const double* zp = A.mem.zpart + ((size_t)b * A.G + g) * 2;
+        const double* zp = A.mem.zpart + ((size_t)b * A.G + g) * 3;
         const double z = zp[0];
         const int kz = (int)zp[1];
+        if constexpr (F == AFF) low = fmax(low, zp[2]);
         const int km = max(zk, kz);
         zm = scale2(zm, max(zk - km, -4000)) + scale2(z, max(kz - km, -4000));
         zk = km;
@@ -548,6 +586,11 @@ __device__ __forceinline__ void element_partition(const Args& A, int b, double& 
         zk += e;
     } else {
         zm = 0.0;
+    }
+    if constexpr (F == AFF) {
+        if (low > -FLT_MAX && !(A.k.oc <= 0.0 && A.k.ec <= 0.0 && zk <= kMaxMaskedExp &&
+                                low + (double)zk <= kNoShare))
+            zm = 0.0;
     }
 }
 
@@ -609,7 +652,7 @@ __global__ void __launch_bounds__((Traits<F>::AFFINE ? 4 : MAXW) * 64) bwd_kerne
     // Z of the element
     double zm = 0.0;
     int zk = -(1 << 28);
-    element_partition(A, b, zm, zk);
+    element_partition<F>(A, b, zm, zk);
     if (!(zm > 0.0) && threadIdx.x == 0) flag_redo(A.redo + b);   // out of range
     const double invZ = 1.0 / zm;
     // S in units of T, from a 64-bit logarithm; every part that reports uses the same
@@ -1305,7 +1348,7 @@ __device__ __forceinline__ void fwd2_sweep(const Args& A, int b, int part) {
             z = scale2(z, max(kz - km, -4000)) + scale2(zred[w], max(kred[w] - km, -4000));
             kz = km;
         }
-        double* zp = A.mem.zpart + ((size_t)b * A.G + part) * 2;
+        double* zp = A.mem.zpart + ((size_t)b * A.G + part) * 3;
         zp[0] = z;
         zp[1] = (double)kz;
     }
@@ -1386,7 +1429,7 @@ __device__ __forceinline__ void bwd2_sweep(const Args& A, int b, int part) {
     // Z of the element
     double zm = 0.0;
     int zk = -(1 << 28);
-    element_partition(A, b, zm, zk);
+    element_partition<F>(A, b, zm, zk);
     if (!(zm > 0.0) && threadIdx.x == 0) flag_redo(A.redo + b);
     float* obase = A.out + (size_t)b * A.L1max * A.L2max;
     zero_padding(obase, L1, L2, A.L1max, A.L2max, blockDim.x, min(s0 * 64, A.L1max),
@@ -1706,7 +1749,7 @@ __device__ __forceinline__ void bwd2_sweep(const Args& A, int b, int part) {
                 r[0] += red[0][w];
                 r[2] += red[1][w];
             }
-        element_partition(A, b, zm, zk);
+        element_partition<F>(A, b, zm, zk);
         finish_part<F>(A, b, part, L1, L2, r,
                        A.T * 0.693147180559945309417 * ((double)zk + log2(zm)));
     }

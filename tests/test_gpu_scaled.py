@@ -162,3 +162,71 @@ def test_strong_scores(cuda, B, L1, L2, T, op):
     got = getattr(d2p_amd, op + "_with_grads")(torch.from_numpy(s).to(cuda), -1.0, T, None)
     want = getattr(O.get("oracle64"), op)(s[:4].astype(np.float64), -1.0, T, None)
     _check([x[:4] for x in got], want, s[:4], (-1.0,), T, tol, op == "soft_nw")
+
+
+def _segments(L1, L2, T, match, penalty):
+    """Matches along the diagonal, everything else and the diagonal's middle cell at the
+    penalty: (local alignment, affine gaps) one path has both halves, through that cell."""
+    s = np.full((L1, L2), penalty, np.float32)
+    for i in range(min(L1, L2)):
+        s[i, i] = match
+    s[min(L1, L2) // 2, min(L1, L2) // 2] = penalty
+    return s
+
+
+@pytest.mark.parametrize("L1,L2", [(60, 60), (60, 250), (300, 310)])
+@pytest.mark.parametrize("T,match,penalty,gaps", [
+    (1.0, 5.0, -80.0, (-11.0, -1.0)),       # factors within the 32-bit range
+    (1.0, 5.0, -90.0, (-11.0, -1.0)),       # below it
+    (1.0, 5.0, -110.0, (-11.0, -1.0)),
+    (0.5, 5.0, -75.0, (-11.0, -1.0)),
+    (0.2, 5.0, -22.0, (-3.0, -0.5)),
+    (0.25, 4.0, -100.0, (-3.0, -0.5)),
+    (0.2, 9.0, -200.0, (-3.0, -0.5)),       # below the 64-bit range
+])
+@pytest.mark.parametrize("op", ["soft_sw_affine", "soft_nw_affine"])
+def test_mismatches_that_have_to_be_crossed(cuda, op, T, match, penalty, gaps, L1, L2):
+    # (local affine alignment has no step from one kind of gap to the other)
+    s, _ = _inputs(3, L1, L2, False)
+    s[0] = _segments(L1, L2, T, match, penalty)
+    s[1, L1 // 2, L2 // 3] = penalty        # a cell that no path has to cross
+    got = getattr(d2p_amd, op + "_with_grads")(torch.from_numpy(s).to(cuda), *gaps, T, None)
+    want = getattr(O.get("oracle64"), op)(s.astype(np.float64), *gaps, T, None)
+    # alpha's rounding, for the elements that the log-domain sweeps take: half an ulp of
+    # the value's size in each of the path's cells, to either side
+    m = min(L1, L2)
+    tol = _tol(s, m, T) + 8.0 * math.sqrt(L1 + L2) * 2.0 ** -24 * float(want[0].max()) / T
+    _check(got, want, s, gaps, T, tol, op == "soft_nw_affine")
+
+
+def _blocks(B, L1, L2, match, masked):
+    """Two blocks, with matches along their diagonals, one more in the second; everything outside
+    of them masked, three rows and columns between them included."""
+    s, _ = _inputs(B, L1, L2, False)
+    c1, c2 = int(0.45 * L1), int(0.45 * L2)
+    n = min(c1, c2) - 3
+    for i in range(n):
+        s[:, i, i] = match
+    for i in range(n + 1):
+        s[:, c1 + i, c2 + i] = match
+    s[:, :c1, c2 - 3:] = masked
+    s[:, c1 - 3:, :c2] = masked
+    return s
+
+
+@pytest.mark.parametrize("T,match", [(1.0, 2.0), (1.0, 8.0), (0.2, 5.0)])
+@pytest.mark.parametrize("masked", [-1e3, -1e9, -1e30])
+@pytest.mark.parametrize("op,gaps", [("soft_sw", (-1.0,)), ("soft_nw", (-1.0,)),
+                                     ("soft_sw_affine", (-3.0, -0.5)),
+                                     ("soft_nw_affine", (-3.0, -0.5))])
+@pytest.mark.parametrize("B,L1,L2", [(2, 190, 160), (300, 190, 160)])
+def test_masked_blocks(cuda, B, L1, L2, op, gaps, masked, T, match):
+    # (local affine alignment: no path has both blocks, and the second one's rows start anew
+    # beside gaps that leave the first one, of weights beyond the 64-bit range above 1)
+    s = _blocks(B, L1, L2, match, masked)
+    got = getattr(d2p_amd, op + "_with_grads")(torch.from_numpy(s).to(cuda), *gaps, T, None)
+    want = getattr(O.get("oracle64"), op)(s[:2].astype(np.float64), *gaps, T, None)
+    live = np.where(s[:2] > -100, s[:2], 0)
+    tol = _tol(live, min(L1, L2), T) + 8.0 * math.sqrt(L1 + L2) * 2.0 ** -24 * float(
+        np.abs(want[0]).max()) / T
+    _check([x[:2] for x in got], want, s[:2], gaps, T, tol, "nw" in op)
