@@ -996,6 +996,15 @@ __global__ void __launch_bounds__((Traits<F>::AFFINE ? 4 : MAXW) * 64) bwd_kerne
             if (full && !(F == NWAFF && !above)) chunk(std::true_type{});
             else chunk(std::false_type{});
             post(prog, wave, q + 1);
+            if (__builtin_amdgcn_ballot_w64(ps != ps) != 0) {
+                // -inf scores, whose marginals are 0: the sum again, of finite scores.  (One test
+                // a chunk; a clamp of every score would be one instruction a cell.)
+                ps = 0.0f;
+#pragma unroll
+                for (int j = P - 1; j >= 0; --j)
+                    ps = fmaf(*reinterpret_cast<const float*>(orow + ((oaddr + 4u * j) & 124u)),
+                              __builtin_amdgcn_fmed3f(scores(j / 4)[j & 3], -FLT_MAX, FLT_MAX), ps);
+            }
             pacc += (double)ps;
             __asm__ volatile("" ::: "memory");
         }

@@ -230,3 +230,20 @@ def test_masked_blocks(cuda, B, L1, L2, op, gaps, masked, T, match):
     tol = _tol(live, min(L1, L2), T) + 8.0 * math.sqrt(L1 + L2) * 2.0 ** -24 * float(
         np.abs(want[0]).max()) / T
     _check([x[:2] for x in got], want, s[:2], gaps, T, tol, "nw" in op)
+
+
+@pytest.mark.parametrize("op,gaps", [("soft_sw", (-1.0,)), ("soft_nw", (-1.0,)),
+                                     ("soft_sw_affine", (-2.0, -0.5)),
+                                     ("soft_nw_affine", (-2.0, -0.5))])
+@pytest.mark.parametrize("B,L1,L2", [(3, 130, 70), (300, 130, 70), (3, 300, 83)])
+def test_infinite_masks_keep_the_sweeps(cuda, B, L1, L2, op, gaps):
+    # the factor of -inf and of -1e30 is 0 alike: the same bits, from the same sweeps
+    out = []
+    for masked in (-1e30, -math.inf):
+        s, _ = _inputs(B, L1, L2, False)
+        s[:, :, 50:60] = masked
+        s[1, 20:, :] = masked
+        out.append(getattr(d2p_amd, op + "_with_grads")(torch.from_numpy(s).to(cuda), *gaps, 1.0,
+                                                        None))
+    for n, (a, b) in enumerate(zip(*out)):
+        assert torch.equal(a, b), (n, float((a - b).abs().max()))
