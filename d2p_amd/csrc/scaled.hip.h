@@ -17,7 +17,8 @@
 //
 // Range.  Scores that move a lane's values up by more than about 60 bits a step take them
 // beyond 2^1023 of its chunk's scale: they become infinite or NaN, which the sweeps detect.
-// They set redo[b], and the log-domain sweeps recompute that element.
+// They set redo[b], the reverse sweep is left out where the forward found it, and the log-domain
+// sweeps recompute that element, in the launch shape that they would have taken.
 // Downwards nothing becomes infinite.  E is 0 below 2^-149 (and rounded below 2^-126), and
 // values below 2^-1022 of the scale are lost.  Where two gaps go round any match (linear
 // gaps, and global affine ones, whose gaps follow each other in either order) they bound both:
@@ -70,7 +71,7 @@ constexpr float kMinBits = -126.0f;
 // local affine elements with smaller factors (element_partition): log2 of Z at most, and log2 of
 // the share of Z of the paths through one such cell at most (2^20 cells: 2^-40 in all)
 constexpr int kMaxMaskedExp = 850;
-constexpr double kNoShare = -60.0;
+constexpr float kNoShare = -60.0f;
 // exponent of the SW scale: below it the restart term 1 would overflow
 constexpr int kMinExp = -900;
 
@@ -197,8 +198,13 @@ struct Ring {
     int pad[RCH];
 };
 
-__device__ __forceinline__ void flag_redo(int* redo_b) {
-    __hip_atomic_store(redo_b, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+// Marks an element for the log-domain sweeps.  The bits tell what the forward found, which every
+// part of the reverse sweep sees, from what a part of the reverse sweep found, which the
+// others may or may not.
+enum { REDO_FWD = 1, REDO_BWD = 2 };
+static_assert((REDO_FWD | REDO_BWD) < 1 << REDO_BITS, "below the count of parts");
+__device__ __forceinline__ void flag_redo(int* redo_b, int bit) {
+    __hip_atomic_fetch_or(redo_b, bit, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 
 // The quads of one chunk of the stripe, clamped only where the 16-byte loads could

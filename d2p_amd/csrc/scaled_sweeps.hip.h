@@ -402,7 +402,7 @@ __global__ void __launch_bounds__(MAXW * 64) fwd_kernel(const Args A) {
         wait_vmcnt<0>();         // (loads into LDS still under way)
         // values out of range
         if (__builtin_amdgcn_ballot_w64(lane_ok && exponent(p[0]) == 1024) != 0 && lane == 0)
-            flag_redo(A.redo + b);
+            flag_redo(A.redo + b, REDO_FWD);
         if constexpr (!Tr::LOCAL) {
             if (owns_end) {
                 zsum = lane == lane_end ? vend : 0.0;
@@ -457,6 +457,8 @@ __global__ void __launch_bounds__(MAXW * 64) fwd_kernel(const Args A) {
         if constexpr (F == AFF) {
             float least = -FLT_MAX;
             for (int w = 0; w < n; ++w) least = fmaxf(least, lred[w]);
+            // (gaps that gain: no bound on what is left out)
+            if (least > -FLT_MAX && (A.k.oc > 0.0 || A.k.ec > 0.0)) least = FLT_MAX;
             zp[2] = (double)least;
         }
     }
@@ -561,7 +563,8 @@ __device__ inline void finalize(const Args& A, int b, int L1, int L2, const doub
 // no detour of two gaps bounds what a factor below 2^kMinBits, which is not kept, would
 // weigh.  Such a factor E may be left out if
 //  * E Z is small: a path through its cell is an alignment before it and one behind it (and
-//    gaps, of at most 1 each), of at most Z each, so its share of Z is at most E Z;
+//    gaps, of at most 1 each where they cost), of at most Z each, so its share of Z is at most
+//    E Z;
 //  * 2^-K, the restart term in the lanes' scale, is within the 64-bit range with room for
 //    another factor (K is at most the exponent of Z, and of Z times the rows in the reverse
 //    sweep): beside a cell without weight nothing else keeps a row from its neighbour's
@@ -570,12 +573,12 @@ template <Fam F>
 __device__ __forceinline__ void element_partition(const Args& A, int b, double& zm, int& zk) {
     zm = 0.0;
     zk = -(1 << 28);
-    double low = -FLT_MAX;
+    float low = -FLT_MAX;
     for (int g = 0; g < A.G; ++g) {
         const double* zp = A.mem.zpart + ((size_t)b * A.G + g) * 3;
         const double z = zp[0];
         const int kz = (int)zp[1];
-        if constexpr (F == AFF) low = fmax(low, zp[2]);
+        if constexpr (F == AFF) low = fmaxf(low, (float)zp[2]);
         const int km = max(zk, kz);
         zm = scale2(zm, max(zk - km, -4000)) + scale2(z, max(kz - km, -4000));
         zk = km;
@@ -588,9 +591,7 @@ __device__ __forceinline__ void element_partition(const Args& A, int b, double& 
         zm = 0.0;
     }
     if constexpr (F == AFF) {
-        if (low > -FLT_MAX && !(A.k.oc <= 0.0 && A.k.ec <= 0.0 && zk <= kMaxMaskedExp &&
-                                low + (double)zk <= kNoShare))
-            zm = 0.0;
+        if (low > -FLT_MAX && (zk > kMaxMaskedExp || low > kNoShare - (float)zk)) zm = 0.0;
     }
 }
 
@@ -599,7 +600,7 @@ template <Fam F>
 __device__ inline void finish_part(const Args& A, int b, int part, int L1, int L2, const double* r,
                                    double S) {
     for (int i = 0; i < 3; ++i)
-        if (exponent(fabs(r[i])) == 1024) flag_redo(A.redo + b);
+        if (exponent(fabs(r[i])) == 1024) flag_redo(A.redo + b, REDO_BWD);
     if (A.G == 1) {
         finalize<F>(A, b, L1, L2, r, S);
     } else {
@@ -653,7 +654,7 @@ __global__ void __launch_bounds__((Traits<F>::AFFINE ? 4 : MAXW) * 64) bwd_kerne
     double zm = 0.0;
     int zk = -(1 << 28);
     element_partition<F>(A, b, zm, zk);
-    if (!(zm > 0.0) && threadIdx.x == 0) flag_redo(A.redo + b);   // out of range
+    if (!(zm > 0.0) && threadIdx.x == 0) flag_redo(A.redo + b, REDO_BWD);   // out of range
     const double invZ = 1.0 / zm;
     // S in units of T, from a 64-bit logarithm; every part that reports uses the same
     const double S = A.T * 0.693147180559945309417 * ((double)zk + log2(zm));
@@ -672,8 +673,8 @@ __global__ void __launch_bounds__((Traits<F>::AFFINE ? 4 : MAXW) * 64) bwd_kerne
     const size_t flow_plane = (size_t)P * nchmax;
     const bool to = n > 0 && s0 > 0, from = n > 0 && s0 + n < NS;
     const int W_IN = A.SPW, W_OUT = A.SPW + 1;
-    // an element already given to the log-domain sweeps needs no reverse sweep here
-    const bool skip = A.G == 1 && __builtin_amdgcn_readfirstlane(A.redo[b]) != 0;
+    // an element given to the log-domain sweeps needs no reverse sweep here (its parts agree)
+    const bool skip = __builtin_amdgcn_readfirstlane(zm > 0.0 ? A.redo[b] & REDO_FWD : 1) != 0;
 
     double gacc = 0.0, hacc = 0.0, pacc = 0.0;   // open (linear: gap), extend, sum of P s
     if (skip) {
@@ -999,11 +1000,16 @@ __global__ void __launch_bounds__((Traits<F>::AFFINE ? 4 : MAXW) * 64) bwd_kerne
             if (__builtin_amdgcn_ballot_w64(ps != ps) != 0) {
                 // -inf scores, whose marginals are 0: the sum again, of finite scores.  (One test
                 // a chunk; a clamp of every score would be one instruction a cell.)
+                int l = lane;
+                __asm__ volatile("" : "+v"(l));   // (rare: nothing of it is kept across chunks)
+                const float* marg = ot->v + 32 * l;
                 ps = 0.0f;
-#pragma unroll
+#pragma unroll 1
                 for (int j = P - 1; j >= 0; --j)
-                    ps = fmaf(*reinterpret_cast<const float*>(orow + ((oaddr + 4u * j) & 124u)),
-                              __builtin_amdgcn_fmed3f(scores(j / 4)[j & 3], -FLT_MAX, FLT_MAX), ps);
+                    ps = fmaf(marg[(t0 - l + OutTile::rot(l) + j) & 31],
+                              __builtin_amdgcn_fmed3f(tile[QuadTile<P>::slot(l, j / 4) + (j & 3)],
+                                                      -FLT_MAX, FLT_MAX),
+                              ps);
             }
             pacc += (double)ps;
             __asm__ volatile("" ::: "memory");
@@ -1277,7 +1283,7 @@ __device__ __forceinline__ void fwd2_sweep(const Args& A, int b, int part) {
         }
         // values out of range
         if (__builtin_amdgcn_ballot_w64(lane_ok && exponent(v) == 1024) != 0 && lane == 0)
-            flag_redo(A.redo + b);
+            flag_redo(A.redo + b, REDO_FWD);
         // the wave's share of the partition
         int km = zk;
 #pragma unroll
@@ -1439,7 +1445,7 @@ __device__ __forceinline__ void bwd2_sweep(const Args& A, int b, int part) {
     double zm = 0.0;
     int zk = -(1 << 28);
     element_partition<F>(A, b, zm, zk);
-    if (!(zm > 0.0) && threadIdx.x == 0) flag_redo(A.redo + b);
+    if (!(zm > 0.0) && threadIdx.x == 0) flag_redo(A.redo + b, REDO_BWD);
     float* obase = A.out + (size_t)b * A.L1max * A.L2max;
     zero_padding(obase, L1, L2, A.L1max, A.L2max, blockDim.x, min(s0 * 64, A.L1max),
                  part == A.G - 1 ? A.L1max : min((s0 + A.SPW) * 64, A.L1max));
@@ -1453,8 +1459,8 @@ __device__ __forceinline__ void bwd2_sweep(const Args& A, int b, int part) {
     const size_t brow_len = (size_t)P * (nchmax + 1);
     const size_t flow_len = (size_t)P * nchmax;
     const bool to = n > 0 && s0 > 0, from = n > 0 && s0 + n < NS;
-    // an element already given to the log-domain sweeps needs no reverse sweep here
-    const bool skip = A.G == 1 && __builtin_amdgcn_readfirstlane(A.redo[b]) != 0;
+    // an element given to the log-domain sweeps needs no reverse sweep here (its parts agree)
+    const bool skip = __builtin_amdgcn_readfirstlane(zm > 0.0 ? A.redo[b] & REDO_FWD : 1) != 0;
 
     if (skip) {
     } else if (wave < n) {
@@ -1791,9 +1797,9 @@ __global__ void __launch_bounds__(3 * ROOMY * 64) both_kernel(const Args A) {
     bwd2_sweep<F>(A, b, 0);
 }
 
-// The end of a split element: sums its parts, or its poison pass.  Called by the kernel that
-// redoes elements out of range, which every call launches: a launch less (NW [96, 301,
-// 277], forward and backward: 186 -> 184 us).
+// The end of a split element that stays here: sums its parts, or its poison pass.  Called by the
+// kernel that redoes elements out of range, which every call launches: a launch less (NW [96,
+// 301, 277], forward and backward: 186 -> 184 us).
 template <Fam F>
 __device__ inline void finish_element(const Args& A, int b) {
     if (A.G == 1) return;
@@ -1813,10 +1819,10 @@ __device__ inline void finish_element(const Args& A, int b) {
 
 static __global__ void reset_kernel(int* __restrict__ status, int* __restrict__ redo,
                              uint64_t* __restrict__ fflag, uint64_t* __restrict__ bflag, int B,
-                             int G) {
+                             int flags) {
     const int i = blockIdx.x * blockDim.x + threadIdx.x;
     if (i < B) status[i] = redo[i] = 0;
-    if (i < B * G) {
+    if (i < flags) {
         store_flag(fflag + i, 0);
         store_flag(bflag + i, 0);
     }
@@ -1904,8 +1910,9 @@ int run(Args& A, void* table, size_t table_bytes, bool* done, hipStream_t st, co
     A.epoch = next_epoch();
     const int copying = sp.G > 1 ? 2 : 0;
     if (sp.G > 1)
-        D2P_LAUNCH("split_reset", reset_kernel, dim3((A.B * sp.G + 255) / 256), dim3(256), 0, st,
-                   A.status, A.redo, A.fflag, A.bflag, A.B, sp.G);
+        // (every word: the sweeps that redo an element may have other parts)
+        D2P_LAUNCH("split_reset", reset_kernel, dim3((A.B * ns + 255) / 256), dim3(256), 0, st,
+                   A.status, A.redo, A.fflag, A.bflag, A.B, A.B * ns);
     const dim3 grid(split_grid(A.B, sp.G));
     void (*fwd)(const Args) = nullptr;
     void (*bwd)(const Args) = bwd_kernel<F>;

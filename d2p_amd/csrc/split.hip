@@ -34,15 +34,7 @@ __global__ void partition_merge_kernel(const float2* __restrict__ fpart,
                                        float* __restrict__ partition, int B, int G, float T) {
     const int b = blockIdx.x * blockDim.x + threadIdx.x;
     if (b >= B) return;
-    const float c = kLog2e / T;
-    OnlineLSE tot;
-    tot.m = 0.0f;
-    tot.z = 1.0f;
-    for (int g = 0; g < G; ++g) {
-        const float2 v = fpart[(size_t)b * G + g];
-        tot.merge(v.x, v.y, c);
-    }
-    partition[b] = tot.m + T * kLn2 * fast_log2(tot.z);
+    partition[b] = merge_partition(fpart + (size_t)b * G, G, T);
 }
 
 __global__ void partition_dot_merge_kernel(const float2* __restrict__ fpart,

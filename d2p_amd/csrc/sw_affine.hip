@@ -22,6 +22,7 @@
 
 #include <vector>
 
+#include <algorithm>
 #include <cstdlib>
 #include <type_traits>
 
@@ -1060,61 +1061,82 @@ swa_backward_kernel(const float* __restrict__ scores, const int* __restrict__ le
                               L1max, L2max, NSmax, go, ge, T, R, G, SPW, epoch);
 }
 
-// After the linear-domain sweeps: the end of split elements, then both log-domain sweeps
-// of the elements that `redo` marks (values out of range), one workgroup each; the
-// others leave at once.
-template <bool NWA>
-__global__ void __launch_bounds__(NW * 64)
-swa_redo_kernel(const sc::Args A, const float* __restrict__ scores,
-                const int* __restrict__ lengths, const Layout ws, float* __restrict__ value,
-                float* __restrict__ post, float* __restrict__ grad_open,
-                float* __restrict__ grad_ext, float* __restrict__ grad_T, int B, int L1max,
-                int L2max, int NSmax, float go, float ge, float T, int Rf, int Rb,
-                uint32_t epoch) {
-    __shared__ int poison_flag;
-    int b, part;
-    split_decode(blockIdx.x, 1, b, part);
-    if (b >= B) return;
-    sc::finish_element<NWA ? sc::NWAFF : sc::AFF>(A, b);
-    if (A.redo[b] == 0) return;
-    __syncthreads();
-    forward_sweep<NWA, false>(scores, lengths, ws.alpha_sk, ws.brow, value, ws.status, ws.fflag,
-                              ws.fpart, B, L1max, L2max, NSmax, go, ge, T, Rf, 1, NSmax, epoch);
-    __threadfence_block();
-    __syncthreads();
-    backward_sweep<NWA, false>(scores, lengths, ws.alpha_sk, ws.brow, value, post, grad_open,
-                               grad_ext, grad_T, ws.status, ws.trash, ws.bflag,
-                               reinterpret_cast<float4*>(ws.flows), nullptr, ws.bpart, B, L1max,
-                               L2max, NSmax, go, ge, T, Rb, 1, NSmax, epoch);
-    // waits that gave up: NaN everywhere
-    wait_vmcnt<0>();
-    __syncthreads();
-    if (threadIdx.x == 0) poison_flag = load_status(ws.status + b);
-    __syncthreads();
-    if (poison_flag == 0) return;
-    const float nan = __builtin_nanf("");
-    const size_t n = (size_t)L1max * L2max;
-    for (size_t i = threadIdx.x; i < n; i += blockDim.x) post[(size_t)b * n + i] = nan;
-    if (threadIdx.x == 0) value[b] = grad_open[b] = grad_ext[b] = grad_T[b] = nan;
+// grad_open[b], grad_ext[b], grad_T[b] of a split element from the parts' sums.
+__device__ __forceinline__ void merge_grads(const double* parts, float S, int G, float go, float ge,
+                                            float T, float* grad_open, float* grad_ext,
+                                            float* grad_T) {
+    float go_s = 0.0f, ge_s = 0.0f, p = 0.0f;
+    for (int i = 0; i < G; ++i) {
+        go_s += (float)parts[4 * i];
+        ge_s += (float)parts[4 * i + 1];
+        p += (float)parts[4 * i + 2];
+    }
+    *grad_open = go_s;
+    *grad_ext = ge_s;
+    *grad_T = (S - (p + (go_s * go + ge_s * ge))) / T;
 }
 
-// grad_open[b], grad_ext[b], grad_T[b] of a split element from the parts' sums.
 __global__ void swa_grad_merge(const double* __restrict__ bpart, const float* __restrict__ partition,
                                float* __restrict__ grad_open, float* __restrict__ grad_ext,
                                float* __restrict__ grad_T, int B, int G, float go, float ge,
                                float T) {
     const int b = blockIdx.x * blockDim.x + threadIdx.x;
     if (b >= B) return;
-    float go_s = 0.0f, ge_s = 0.0f, p = 0.0f;
-    for (int i = 0; i < G; ++i) {
-        const double* bp = bpart + ((size_t)b * G + i) * 4;
-        go_s += (float)bp[0];
-        ge_s += (float)bp[1];
-        p += (float)bp[2];
+    merge_grads(bpart + (size_t)b * G * 4, partition[b], G, go, ge, T, grad_open + b, grad_ext + b,
+                grad_T + b);
+}
+
+// After the linear-domain sweeps: the end of split elements, then both log-domain sweeps
+// of the elements that `redo` marks (values out of range), as for linear gaps: in the parts
+// and with the helper waves that these sweeps have by themselves, parts meeting between the
+// sweeps, their sums in the element's flows of stripe 0, which no part reads.
+// With every element of the call marked, microseconds per call (linear-domain sweeps before it
+// included; the log-domain sweeps alone; one unsplit workgroup without helpers an element):
+//   local [32, 500, 450]       731    564   1093
+//   local [2, 1000, 1000]     1502   1163   2940
+//   global [32, 500, 450]      976    805   1337
+template <bool NWA, bool HELP>
+__global__ void __launch_bounds__(NW * 64)
+swa_redo_kernel(const sc::Args A, const float* __restrict__ scores,
+                const int* __restrict__ lengths, const Layout ws, float* __restrict__ value,
+                float* __restrict__ post, float* __restrict__ grad_open,
+                float* __restrict__ grad_ext, float* __restrict__ grad_T, int B, int L1max,
+                int L2max, int NSmax, float go, float ge, float T, int Rf, int Rb, int G, int SPW,
+                uint32_t epoch_f, uint32_t epoch_b) {
+    __shared__ int last;
+    int b, part;
+    split_decode(blockIdx.x, G, b, part);
+    if (b >= B) return;
+    if ((A.redo[b] & (sc::REDO_FWD | sc::REDO_BWD)) == 0) {
+        if (part == 0) sc::finish_element<NWA ? sc::NWAFF : sc::AFF>(A, b);
+        return;
     }
-    grad_open[b] = go_s;
-    grad_ext[b] = ge_s;
-    grad_T[b] = (partition[b] - (p + (go_s * go + ge_s * ge))) / T;
+    float4* flows4 = reinterpret_cast<float4*>(ws.flows);
+    float* flows1 = G > 1 ? reinterpret_cast<float*>(flows4 + ws.flow_slots) : nullptr;
+    double* sums = reinterpret_cast<double*>(flows4 + (size_t)b * NSmax * stored_steps(L2max));
+    float2* fsums = reinterpret_cast<float2*>(sums + 4 * G);
+    const size_t first = (size_t)b * G;
+    forward_sweep<NWA, HELP>(scores, lengths, ws.alpha_sk, ws.brow, value, ws.status, ws.fflag,
+                             fsums - first, B, L1max, L2max, NSmax, go, ge, T, Rf, G, SPW,
+                             epoch_f);
+    if (G > 1) {
+        wait_all_parts(ws.fflag + first, G, part, epoch_f, L2max + 64, ws.status + b);
+        if (!NWA && threadIdx.x == 0) value[b] = merge_partition(fsums, G, T);
+    }
+    wait_vmcnt<0>();
+    __threadfence_block();
+    __syncthreads();
+    backward_sweep<NWA, HELP>(scores, lengths, ws.alpha_sk, ws.brow, value, post, grad_open,
+                              grad_ext, grad_T, ws.status, ws.trash, ws.bflag, flows4, flows1,
+                              sums - 4 * first, B, L1max, L2max, NSmax, go, ge, T, Rb, G, SPW,
+                              epoch_b);
+    if (!last_part(A.redo + b, G, &last)) return;
+    if (G > 1 && threadIdx.x == 0)
+        merge_grads(sums, value[b], G, go, ge, T, grad_open + b, grad_ext + b, grad_T + b);
+    __syncthreads();
+    // waits that gave up: NaN everywhere
+    if (__builtin_amdgcn_readfirstlane(load_status(ws.status + b)) != 0)
+        sc::poison<NWA ? sc::NWAFF : sc::AFF>(A, b);
 }
 
 }  // namespace swa
@@ -1133,6 +1155,8 @@ size_t lds_forward_r(int R) {
     return (size_t)NW * (2 * 64 * PF + 2 * 3 * 64) * sizeof(float) +
            ((size_t)NW * R + NW * DUMMY) * sizeof(float4);
 }
+// ... and with helper waves, for the odd chunks' M and I tiles after the rings
+size_t lds_forward_help() { return (size_t)(NW / 2) * 2 * PF * 64 * sizeof(float); }
 size_t lds_backward_r(int R, bool nwa) {
     const size_t tile = (nwa ? 65 : 64) * PB;   // dword or quad tiles
     const size_t wfloats = tile + 3 * PB * 64 + 3 * 64 + tile + 2 * 64;
@@ -1184,10 +1208,9 @@ int launch_forward(const float* scores, const int* lengths, int B, int max_L1, i
     size_t lds = lds_forward_r(R);
     D2P_REQUIRE(lds <= kLdsLimit, "sequence too long for the LDS stripe rings");
     if (sp.G > 1 && launch_split_reset(ws, B, sp.G, st) != D2P_OK) return D2P_ERR_HIP;
-    // helper waves (local form, parts of at most NW/2 stripes) need the odd chunks' M
-    // and I tiles after the rings: NW/2 x 2P x 64 floats
+    // helper waves: local form, parts of at most NW/2 stripes
     const int part_stripes = sp.G > 1 ? sp.SPW : ns;
-    const size_t lds_help = lds + (size_t)(NW / 2) * 2 * PF * 64 * sizeof(float);
+    const size_t lds_help = lds + lds_forward_help();
     const bool help =
         !nwa && part_stripes <= NW / 2 && lds_help <= kLdsLimit && helpers_enabled();
     if (help) lds = lds_help;
@@ -1241,25 +1264,56 @@ int launch_backward(const float* scores, const int* lengths, int B, int max_L1, 
     return D2P_OK;
 }
 
-// LDS of the two log-domain sweeps of an unsplit element in one workgroup (the second
-// one's static arrays come on top)
-size_t redo_lds(int max_L1, int max_L2, bool nwa) {
-    const size_t f = lds_forward_r(ring_forward(max_L1, max_L2));
-    const size_t b = lds_backward_r(ring_backward(max_L1, max_L2), nwa);
-    return (f > b ? f : b) + 1024;
+// LDS that one launch of both log-domain sweeps may take beside the static arrays of both
+constexpr size_t kRedoLds = kLdsLimit - 1024;
+
+// Its shape, as for linear gaps: the parts that the sweeps have by themselves where all of them
+// are resident and `split` (the linear-domain sweeps have reset the progress words), else
+// one workgroup an element.
+struct RedoShape {
+    Split sp;
+    int Rf, Rb;
+    bool help;
+    size_t lds;
+};
+RedoShape redo_shape(int B, int max_L1, int max_L2, const Layout& ws, bool nwa, bool split) {
+    RedoShape r;
+    const int ns = (max_L1 + 63) / 64;
+    r.sp = Split{1, ns > 0 ? ns : 1};
+    if (split) {
+        const Split sp =
+            choose_split(B, max_L1, ws, std::max(max_stripes_forward(max_L1, max_L2),
+                                                 max_stripes_backward(max_L1, max_L2, nwa)));
+        const size_t sums = (size_t)sp.G * (4 * sizeof(double) + sizeof(float2));
+        if (split_grid(B, sp.G) <= device_cus() &&
+            sums <= (size_t)stored_steps(max_L2) * sizeof(float4))
+            r.sp = sp;
+    }
+    const int rows = r.sp.G > 1 ? r.sp.SPW * 64 : max_L1;
+    r.Rf = ring_forward(rows, max_L2);
+    r.Rb = ring_backward(rows, max_L2);
+    size_t f = lds_forward_r(r.Rf);
+    const size_t f_help = f + lds_forward_help();
+    r.help = !nwa && (rows + 63) / 64 <= NW / 2 && f_help <= kRedoLds && helpers_enabled();
+    if (r.help) f = f_help;
+    r.lds = std::max(f, lds_backward_r(r.Rb, nwa));
+    return r;
 }
 
-int launch_redo(const sc::Args& args, const float* scores, const int* lengths, int B, int max_L1, int max_L2, float go,
-                float ge, float T, const Layout& ws, float* value, float* marginals,
-                float* grad_open, float* grad_ext, float* grad_T, hipStream_t st, bool nwa) {
-    const size_t lds = redo_lds(max_L1, max_L2, nwa) - 1024;
-    auto k = nwa ? swa_redo_kernel<true> : swa_redo_kernel<false>;
+int launch_redo(const sc::Args& args, const float* scores, const int* lengths, int B, int max_L1,
+                int max_L2, float go, float ge, float T, const Layout& ws, float* value,
+                float* marginals, float* grad_open, float* grad_ext, float* grad_T, hipStream_t st,
+                bool nwa) {
+    const RedoShape r = redo_shape(B, max_L1, max_L2, ws, nwa, args.G > 1);
+    auto k = nwa ? swa_redo_kernel<true, false>
+                 : r.help ? swa_redo_kernel<false, true> : swa_redo_kernel<false, false>;
     D2P_HIP(hipFuncSetAttribute((const void*)k, hipFuncAttributeMaxDynamicSharedMemorySize,
-                                (int)lds));
-    D2P_LAUNCH(nwa ? "nwa_redo" : "swa_redo", k, dim3(split_grid(B, 1)), dim3(NW * 64), lds, st,
-               args, scores, lengths, ws, value, marginals, grad_open, grad_ext, grad_T, B,
-               max_L1, max_L2, (max_L1 + 63) / 64, go, ge, T, ring_forward(max_L1, max_L2),
-               ring_backward(max_L1, max_L2), next_epoch());
+                                (int)r.lds));
+    const uint32_t epoch_f = next_epoch(), epoch_b = next_epoch();
+    D2P_LAUNCH(nwa ? "nwa_redo" : "swa_redo", k, dim3(split_grid(B, r.sp.G)), dim3(NW * 64), r.lds,
+               st, args, scores, lengths, ws, value, marginals, grad_open, grad_ext, grad_T, B,
+               max_L1, max_L2, (max_L1 + 63) / 64, go, ge, T, r.Rf, r.Rb, r.sp.G, r.sp.SPW,
+               epoch_f, epoch_b);
     D2P_HIP(hipGetLastError());
     return D2P_OK;
 }
@@ -1293,7 +1347,7 @@ int affine_forward_marginals(const float* scores, const int* lengths, int B, int
     const wf::Layout ws = swa::affine_layout(workspace, B, max_L1, max_L2, true);
     bool done = false;
     sc::Args args;
-    if (swa::redo_lds(max_L1, max_L2, nwa) <= swa::kLdsLimit)
+    if (swa::redo_shape(B, max_L1, max_L2, ws, nwa, false).lds <= swa::kRedoLds)
         D2P_TRY(swa::run_scaled(scores, lengths, B, max_L1, max_L2, gap_open, gap_ext, temperature,
                                 ws, value, marginals, grad_open, grad_ext, grad_T, st, nwa, &done,
                                 &args));

@@ -17,6 +17,7 @@
 // previous step, in the reference's accumulation order
 //   beta = ((beta_init + from(i+1,j+1)) + from(i,j+1)) + from(i+1,j).
 
+#include <algorithm>
 #include <atomic>
 #include <cstdlib>
 #include <mutex>
@@ -1486,34 +1487,74 @@ sw_backward_kernel(const float* __restrict__ scores, const int* __restrict__ len
         flows, bpart, poison_value, B, L1max, L2max, NSmax, gap, T, R, G, SPW, epoch);
 }
 
+// grad_gap[b], grad_T[b] of a split element from the parts' sums.
+template <typename Acc>
+__device__ __forceinline__ void merge_grads(const double* parts, float S, int G, float gap,
+                                            float T, float* grad_gap, float* grad_T) {
+    Acc g = 0, p = 0;
+    for (int i = 0; i < G; ++i) {
+        g += (Acc)parts[2 * i];
+        p += (Acc)parts[2 * i + 1];
+    }
+    *grad_gap = (float)g;
+    *grad_T = (float)(((Acc)S - (p + g * (Acc)gap)) / (Acc)T);
+}
+
 // After the linear-domain sweeps: the end of split elements, then both log-domain sweeps
-// of the elements that `redo` marks (values out of range), one workgroup each; the
-// others leave at once.  One launch, so that a call without such elements, which is nearly every call, pays for one empty grid
-// (3 us) and not for two.
-template <bool NWG>
-__global__ void __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(1, 2)))
+// of the elements that `redo` marks (values out of range), in the parts and with the helper
+// waves that these sweeps have by themselves; the other elements leave at once.  One launch, so
+// that a call without such elements, which is nearly every call, pays for one empty grid (3 us)
+// and not for two.
+// Split elements (G > 1) meet between the sweeps (wait_all_parts), and the last part to end adds
+// them up.  Their sums lie in the element's flows of stripe 0, which no part reads:
+// A.bpart and A.redo (= ws.fpart) are other elements' still.
+// With every element of the call marked, microseconds per call (linear-domain sweeps before it
+// included; the log-domain sweeps alone; one unsplit workgroup without helpers an element):
+//   SW [2, 1000, 1000]      727    566   1540
+//   SW [256, 512, 512]      479    376    642
+//   SW [64, 384, 384]       306    222    434
+//   NW [96, 301, 277]       363    254    380
+template <bool NWG, bool HELP, bool WIDE, int P>
+__global__ void __launch_bounds__(WIDE ? 2 * NW * 64 : NW * 64)
+__attribute__((amdgpu_waves_per_eu(WIDE ? 4 : 1, WIDE ? 4 : 2)))
 sw_redo_kernel(const sc::Args A, const float* __restrict__ scores,
                const int* __restrict__ lengths, const Layout ws, float* __restrict__ value,
                float* __restrict__ post, float* __restrict__ grad_gap, float* __restrict__ grad_T,
-               int B, int L1max, int L2max, int NSmax, float gap, float T, int Rf, int Rb,
-               uint32_t epoch) {
+               int B, int L1max, int L2max, int NSmax, float gap, float T, int Rf, int Rb, int G,
+               int SPW, uint32_t epoch_f, uint32_t epoch_b) {
+    __shared__ int last;
     int b, part;
-    split_decode(blockIdx.x, 1, b, part);
+    split_decode(blockIdx.x, G, b, part);
     if (b >= B) return;
-    sc::finish_element<NWG ? sc::NW : sc::SW>(A, b);
-    if (A.redo[b] == 0) return;
-    __syncthreads();
-    forward_sweep<NWG, false, false, false>(scores, lengths, ws.alpha_sk, ws.brow, value, ws.status,
-                                            ws.fflag, ws.fpart, B, L1max, L2max, NSmax, gap, T, Rf,
-                                            1, NSmax, epoch, 0, TanArgs{});
+    if ((A.redo[b] & (sc::REDO_FWD | sc::REDO_BWD)) == 0) {
+        if (part == 0) sc::finish_element<NWG ? sc::NW : sc::SW>(A, b);
+        return;
+    }
+    double* sums = reinterpret_cast<double*>(ws.flows + (size_t)b * NSmax * stored_steps(L2max));
+    float2* fsums = reinterpret_cast<float2*>(sums + 2 * G);
+    const size_t first = (size_t)b * G;
+    forward_sweep<NWG, HELP, WIDE, false>(scores, lengths, ws.alpha_sk, ws.brow, value, ws.status,
+                                          ws.fflag, fsums - first, B, L1max, L2max, NSmax, gap, T,
+                                          Rf, G, SPW, epoch_f, 0, TanArgs{});
+    if (G > 1) {
+        wait_all_parts(ws.fflag + first, G, part, epoch_f, L2max + 64, ws.status + b);
+        if (!NWG && threadIdx.x == 0) value[b] = merge_partition(fsums, G, T);
+    }
+    wait_vmcnt<0>();
     __threadfence_block();
     __syncthreads();
-    backward_sweep<8, false, NWG, false, false, false>(
+    constexpr bool HELPB = HELP && !NWG;
+    backward_sweep<P, false, NWG, HELPB, HELPB && WIDE, false>(
         scores, lengths, ws.alpha_sk, ws.brow, value, post, grad_gap, grad_T, ws.status, ws.trash,
-        ws.bflag, ws.flows, ws.bpart, value, B, L1max, L2max, NSmax, gap, T, Rb, 1, NSmax, epoch);
+        ws.bflag, ws.flows, sums - 2 * first, G == 1 ? value : nullptr, B, L1max, L2max, NSmax,
+        gap, T, Rb, G, SPW, epoch_b);
+    if (G == 1 || !last_part(A.redo + b, G, &last)) return;
+    if (threadIdx.x == 0) merge_grads<float>(sums, value[b], G, gap, T, grad_gap + b, grad_T + b);
+    __syncthreads();
+    if (__builtin_amdgcn_readfirstlane(load_status(ws.status + b)) != 0)
+        sc::poison<NWG ? sc::NW : sc::SW>(A, b);
 }
 
-// grad_gap[b], grad_T[b] of a split element from the parts' sums.
 template <bool PRECISE>
 __global__ void sw_grad_merge(const double* __restrict__ bpart, const float* __restrict__ partition,
                               float* __restrict__ grad_gap, float* __restrict__ grad_T, int B,
@@ -1521,13 +1562,7 @@ __global__ void sw_grad_merge(const double* __restrict__ bpart, const float* __r
     using Acc = typename std::conditional<PRECISE, double, float>::type;
     const int b = blockIdx.x * blockDim.x + threadIdx.x;
     if (b >= B) return;
-    Acc g = 0, p = 0;
-    for (int i = 0; i < G; ++i) {
-        g += (Acc)bpart[((size_t)b * G + i) * 2];
-        p += (Acc)bpart[((size_t)b * G + i) * 2 + 1];
-    }
-    grad_gap[b] = (float)g;
-    grad_T[b] = (float)(((Acc)partition[b] - (p + g * (Acc)gap)) / (Acc)T);
+    merge_grads<Acc>(bpart + (size_t)b * G * 2, partition[b], G, gap, T, grad_gap + b, grad_T + b);
 }
 
 }  // namespace sw
@@ -1779,27 +1814,60 @@ int launch_backward(const float* scores, const int* lengths, int B, int max_L1, 
 #undef D2P_SW_BWD
 }
 
-// LDS of the two log-domain sweeps of an unsplit element in one workgroup (8-step reverse
-// chunks, which fit longer rows than 16-step ones); the second one's static arrays come on top
-size_t redo_lds(int max_L1, int max_L2) {
-    const size_t f = lds_forward_r(ring_forward(max_L1, max_L2));
-    const size_t b = lds_backward_r(ring_backward(max_L1, max_L2), 8);
-    return (f > b ? f : b) + 1024;
+// LDS that one launch of both log-domain sweeps may take beside the static arrays of both
+constexpr size_t kRedoLds = kLdsLimit - 1024;
+
+// Its shape: the parts that the sweeps have by themselves where all of them are resident, as
+// they wait for each other between the sweeps, and where `split` (the linear-domain sweeps
+// have reset the progress words); else one workgroup an element.
+struct RedoShape {
+    Split sp;
+    int Rf, Rb, P;
+    bool help, wide;
+    size_t lds;
+};
+RedoShape redo_shape(int B, int max_L1, int max_L2, const Layout& ws, bool global, bool split) {
+    RedoShape r;
+    const int ns = (max_L1 + 63) / 64;
+    r.sp = Split{1, ns > 0 ? ns : 1};
+    if (split) {
+        const Split sp = choose_split(B, max_L1, ws, std::max(max_stripes_forward(max_L1, max_L2),
+                                                              max_stripes_backward(max_L1, max_L2)));
+        const size_t sums = (size_t)sp.G * (2 * sizeof(double) + sizeof(float2));
+        if (wf::split_grid(B, sp.G) <= device_cus() &&
+            sums <= (size_t)wf::stored_steps(max_L2) * sizeof(float2))
+            r.sp = sp;
+    }
+    const int rows = r.sp.G > 1 ? r.sp.SPW * 64 : max_L1, stripes = (rows + 63) / 64;
+    r.Rf = ring_forward(rows, max_L2);
+    r.Rb = ring_backward(rows, max_L2);
+    r.P = lds_backward_r(r.Rb, 16) <= kRedoLds ? 16 : 8;
+    r.help = r.P == 16 && stripes <= wf::NW / 2 && helpers_enabled();
+    r.wide = !global && r.P == 16 && !r.help && stripes <= wf::NW && helpers_enabled() &&
+             lds_forward_r(r.Rf, 4) <= kRedoLds;
+    r.lds = std::max(lds_forward_r(r.Rf, r.wide ? 4 : 2), lds_backward_r(r.Rb, r.P));
+    return r;
 }
 
-int launch_redo(const sc::Args& args, const float* scores, const int* lengths, int B, int max_L1, int max_L2, float gap,
-                float T, const Layout& ws, float* value, float* marginals, float* grad_gap,
-                float* grad_T, hipStream_t st, bool global) {
-    const size_t lds = redo_lds(max_L1, max_L2) - 1024;
-    void (*k)(const sc::Args, const float*, const int*, const Layout, float*, float*, float*, float*,
-              int, int, int, int, float, float, int, int, uint32_t) =
-        global ? sw_redo_kernel<true> : sw_redo_kernel<false>;
+int launch_redo(const sc::Args& args, const float* scores, const int* lengths, int B, int max_L1,
+                int max_L2, float gap, float T, const Layout& ws, float* value, float* marginals,
+                float* grad_gap, float* grad_T, hipStream_t st, bool global) {
+    const RedoShape r = redo_shape(B, max_L1, max_L2, ws, global, args.G > 1);
+    auto k = sw_redo_kernel<false, false, false, 8>;
+    if (global)
+        k = r.help ? sw_redo_kernel<true, true, false, 16>
+                   : r.P == 16 ? sw_redo_kernel<true, false, false, 16>
+                               : sw_redo_kernel<true, false, false, 8>;
+    else if (r.help) k = sw_redo_kernel<false, true, false, 16>;
+    else if (r.wide) k = sw_redo_kernel<false, true, true, 16>;
+    else if (r.P == 16) k = sw_redo_kernel<false, false, false, 16>;
     D2P_HIP(hipFuncSetAttribute((const void*)k, hipFuncAttributeMaxDynamicSharedMemorySize,
-                                (int)lds));
-    D2P_LAUNCH(global ? "nw_redo" : "sw_redo", k, dim3(wf::split_grid(B, 1)), dim3(wf::NW * 64),
-               lds, st, args, scores, lengths, ws, value, marginals, grad_gap, grad_T, B,
-               max_L1, max_L2, (max_L1 + 63) / 64, gap, T, ring_forward(max_L1, max_L2),
-               ring_backward(max_L1, max_L2), next_epoch());
+                                (int)r.lds));
+    const uint32_t epoch_f = next_epoch(), epoch_b = next_epoch();
+    D2P_LAUNCH(global ? "nw_redo" : "sw_redo", k, dim3(wf::split_grid(B, r.sp.G)),
+               dim3((r.wide ? 2 : 1) * wf::NW * 64), r.lds, st, args, scores, lengths, ws, value,
+               marginals, grad_gap, grad_T, B, max_L1, max_L2, (max_L1 + 63) / 64, gap, T, r.Rf,
+               r.Rb, r.sp.G, r.sp.SPW, epoch_f, epoch_b);
     D2P_HIP(hipGetLastError());
     return D2P_OK;
 }
@@ -1837,7 +1905,7 @@ int first_order(const float* scores, const int* lengths, int B, int max_L1, int 
                 float* grad_T, hipStream_t st, bool global) {
     bool done = false;
     sc::Args args;
-    if (sw::redo_lds(max_L1, max_L2) <= sw::kLdsLimit)
+    if (sw::redo_shape(B, max_L1, max_L2, ws, global, false).lds <= sw::kRedoLds)
         D2P_TRY(sw::run_scaled(scores, lengths, B, max_L1, max_L2, gap, T, ws, value, marginals,
                                grad_gap, grad_T, st, global, &done, &args));
     if (done)

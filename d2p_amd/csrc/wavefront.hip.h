@@ -315,6 +315,53 @@ __device__ __forceinline__ int wait_part(const uint64_t* flag, uint32_t epoch, i
     }
 }
 
+// Partition of an element from its parts' (max, scaled sum) and the cell (0, 0).
+__device__ __forceinline__ float merge_partition(const float2* parts, int G, float T) {
+    const float c = kLog2e / T;
+    OnlineLSE tot;
+    tot.m = 0.0f;
+    tot.z = 1.0f;
+    for (int g = 0; g < G; ++g) tot.merge(parts[g].x, parts[g].y, c);
+    return tot.m + T * kLn2 * fast_log2(tot.z);
+}
+
+// Both sweeps of split elements in one launch.  Between them every part waits for the
+// element's other parts, whose tables and sums it is about to read: what a part has stored is
+// written back to memory (a release of device scope) before its progress word says so, and
+// caches are invalidated (an acquire) behind the wait, so it does not matter which XCDs
+// the parts run on.  All parts have to be resident (the host checks).  `word`: a progress
+// count that the sweep before does not report.
+__device__ __forceinline__ void wait_all_parts(uint64_t* flags, int G, int part, uint32_t epoch,
+                                               int word, int* status_b) {
+    __asm__ volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        __threadfence();
+        store_flag(flags + part, progress_word(epoch, word));
+    }
+    if (threadIdx.x < 64)
+        for (int g = 0; g < G; ++g) wait_part(flags + g, epoch, word, status_b);
+    __syncthreads();
+    __threadfence();
+}
+
+// Counts the parts of an element that get here, above the low REDO_BITS of *counter; true (in
+// every thread) in the last one, which may then read what the others have stored.
+constexpr int REDO_BITS = 2;
+__device__ __forceinline__ bool last_part(int* counter, int G, int* shared) {
+    __asm__ volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        __threadfence();
+        const int old = __hip_atomic_fetch_add(counter, 1 << REDO_BITS, __ATOMIC_RELAXED,
+                                               __HIP_MEMORY_SCOPE_AGENT);
+        *shared = (old >> REDO_BITS) == G - 1;
+    }
+    __syncthreads();
+    __threadfence();
+    return *shared != 0;
+}
+
 // ---------------------------------------------------------------- progress flags
 
 // Progress flags live in LDS.  The writer completes its LDS writes (ring data)

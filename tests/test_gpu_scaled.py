@@ -130,6 +130,69 @@ def test_elements_out_of_range(cuda, L1, L2, op, gaps):
     assert np.all(np.abs(v - want[0]) <= 1e-5 * np.abs(want[0]) + 1e-5), (v, want[0])
 
 
+@pytest.mark.parametrize("op,gaps", [("soft_sw", (-1.0,)), ("soft_nw", (-1.0,)),
+                                     ("soft_sw_affine", (-2.0, -0.5)),
+                                     ("soft_nw_affine", (-2.0, -0.5))])
+@pytest.mark.parametrize("B,L1,L2,parts", [
+    (3, 700, 90, 0),     # both: parts of at most four stripes
+    (3, 300, 83, 5),     # one stripe a part
+    (3, 600, 40, 1),     # log-domain sweeps of ten stripes in one workgroup
+    (70, 1000, 40, 0),   # parts of eight stripes
+    (300, 450, 30, 0),   # eight stripes, unsplit
+    (20, 500, 66, 0),
+    (3, 1000, 1, 0),
+])
+def test_elements_out_of_range_in_every_shape(cuda, monkeypatch, B, L1, L2, parts, op, gaps):
+    # the shapes that the log-domain sweeps have for themselves; element 1 is out of range (and
+    # ragged), and so is the last one
+    if parts:
+        monkeypatch.setenv("D2P_AMD_SPLIT", str(parts))
+    s, _ = _inputs(B, L1, L2, False)
+    lengths = np.full((B, 2), (L1, L2), np.int32)
+    lengths[1] = L1 - 70, L2 - L2 // 3
+    for b in (1, B - 1):
+        s[b, L1 // 2, L2 // 2] = 300.0
+    x, lt = torch.from_numpy(s).to(cuda), torch.from_numpy(lengths).to(cuda)
+    f = getattr(d2p_amd, op + "_with_grads")
+    got = f(x, *gaps, 1.0, lt)
+    idx = [0, 1, B - 1]
+    want = getattr(O.get("oracle64"), op)(s[idx].astype(np.float64), *gaps, 1.0, lengths[idx])
+    tol = _tol(np.clip(s[0], -10, 10), min(L1, L2), 1.0)
+    for i, b in enumerate(idx):
+        # (alpha's rounding, ulp(512) and over T, along the path)
+        _check([v[b:b + 1] for v in got], [w[i:i + 1] for w in want], s[b:b + 1], gaps, 1.0,
+               tol if b == 0 else math.sqrt(L1 + L2) * 2.0 ** -15, "nw" in op)
+    for _ in range(3):
+        again = f(x, *gaps, 1.0, lt)
+        for a, b in zip(got, again):
+            assert torch.equal(a, b)
+
+
+@pytest.mark.parametrize("op,gaps", [("soft_sw", (-1.0,)), ("soft_nw", (-1.0,)),
+                                     ("soft_sw_affine", (-2.0, -0.5)),
+                                     ("soft_nw_affine", (-2.0, -0.5))])
+def test_elements_out_of_range_in_a_graph(cuda, op, gaps):
+    # a replay has the progress words, and the epochs in them, of the one before
+    f = getattr(d2p_amd, op + "_with_grads")
+    inputs = []
+    for seed in range(4):
+        s = np.random.default_rng(seed).standard_normal((3, 700, 90)).astype(np.float32)
+        s[seed % 3, 350, 40] = 300.0
+        inputs.append(torch.from_numpy(s).to(cuda))
+    want = [f(x, *gaps, 1.0, None) for x in inputs]
+    static = inputs[0].clone()
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        got = f(static, *gaps, 1.0, None)
+    for i in (0, 1, 2, 3, 3, 1):
+        static.copy_(inputs[i])
+        graph.replay()
+        torch.cuda.synchronize()
+        for a, b in zip(got, want[i]):
+            assert torch.equal(a, b), i
+
+
 @pytest.mark.parametrize("B,L1,L2", [(300, 130, 66), (40, 300, 200)])
 def test_affine_calls_repeat_bit_for_bit(cuda, B, L1, L2):
     # a wave reads its first chunks' scores only once they have arrived: workgroups that
