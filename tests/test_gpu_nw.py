@@ -18,6 +18,7 @@ import pytest
 import torch
 
 import _capi
+from _sweeps import SWEEPS, in_units
 from oracle import oracle as O
 
 pytestmark = pytest.mark.gpu
@@ -67,9 +68,10 @@ CASES = [
 ]
 
 
+@pytest.mark.parametrize("sweeps", SWEEPS)
 @pytest.mark.parametrize("seed,B,L1,L2,gap,T", CASES)
-def test_nw_matches_oracle(cuda, seed, B, L1, L2, gap, T):
-    s = _seeded(seed, (B, L1, L2))
+def test_nw_matches_oracle(cuda, seed, B, L1, L2, gap, T, sweeps):
+    s, (gap,), T = in_units(sweeps, _seeded(seed, (B, L1, L2)), (gap,), T)
     gpu = _capi.nw_forward_marginals(s.to(cuda), None, gap, T)
     torch.cuda.synchronize()
     _check(gpu, s.numpy(), gap, T)
@@ -87,23 +89,25 @@ def test_nw_ragged_and_empty(cuda):
     assert v[1] == pytest.approx(40 * -0.7) and v[2] == pytest.approx(70 * -0.7) and v[3] == 0.0
 
 
+@pytest.mark.parametrize("sweeps", SWEEPS)
 @pytest.mark.parametrize("n", [2, 3, 11])
-def test_nw_split_parts(cuda, parts, n):
+def test_nw_split_parts(cuda, parts, n, sweeps):
     parts(n)
-    s = _seeded(30 + n, (2, 700, 90))
-    gpu = _capi.nw_forward_marginals(s.to(cuda), None, -1.0, 1.0)
+    s, (gap,), T = in_units(sweeps, _seeded(30 + n, (2, 700, 90)), (-1.0,), 1.0)
+    gpu = _capi.nw_forward_marginals(s.to(cuda), None, gap, T)
     torch.cuda.synchronize()
-    _check(gpu, s.numpy(), -1.0, 1.0)
+    _check(gpu, s.numpy(), gap, T)
 
 
-def test_nw_split_ragged(cuda, parts):
+@pytest.mark.parametrize("sweeps", SWEEPS)
+def test_nw_split_ragged(cuda, parts, sweeps):
     parts(4)
-    s = _seeded(40, (5, 700, 110))
+    s, (gap,), T = in_units(sweeps, _seeded(40, (5, 700, 110)), (-1.0,), 0.7)
     lens = [[700, 110], [0, 40], [193, 0], [1, 1], [257, 81]]
     gpu = _capi.nw_forward_marginals(s.to(cuda), torch.tensor(lens, dtype=torch.int32).to(cuda),
-                                     -1.0, 0.7)
+                                     gap, T)
     torch.cuda.synchronize()
-    _check(gpu, s.numpy(), -1.0, 0.7, lens)
+    _check(gpu, s.numpy(), gap, T, lens)
 
 
 @pytest.mark.parametrize("n", [0, 1])

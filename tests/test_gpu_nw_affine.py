@@ -20,6 +20,7 @@ import torch
 
 import _capi
 from _parity import close_entrywise
+from _sweeps import SWEEPS, in_units
 from oracle import oracle as O
 
 pytestmark = pytest.mark.gpu
@@ -72,9 +73,10 @@ CASES = [
 ]
 
 
+@pytest.mark.parametrize("sweeps", SWEEPS)
 @pytest.mark.parametrize("seed,B,L1,L2,go,ge,T", CASES)
-def test_nwa_matches_oracle(cuda, seed, B, L1, L2, go, ge, T):
-    s = _seeded(seed, (B, L1, L2))
+def test_nwa_matches_oracle(cuda, seed, B, L1, L2, go, ge, T, sweeps):
+    s, (go, ge), T = in_units(sweeps, _seeded(seed, (B, L1, L2)), (go, ge), T)
     gpu = _capi.nwa_forward_marginals(s.to(cuda), None, go, ge, T)
     torch.cuda.synchronize()
     _check(gpu, s.numpy(), go, ge, T)
@@ -95,23 +97,25 @@ def test_nwa_ragged_and_empty(cuda):
     assert (g_o[1], g_e[1], g_o[2], g_e[2], g_o[3], g_e[3]) == (1, 39, 1, 69, 0, 0)
 
 
+@pytest.mark.parametrize("sweeps", SWEEPS)
 @pytest.mark.parametrize("n", [2, 3, 11])
-def test_nwa_split_parts(cuda, parts, n):
+def test_nwa_split_parts(cuda, parts, n, sweeps):
     parts(n)
-    s = _seeded(30 + n, (2, 700, 90))
-    gpu = _capi.nwa_forward_marginals(s.to(cuda), None, -2.0, -0.5, 1.0)
+    s, (go, ge), T = in_units(sweeps, _seeded(30 + n, (2, 700, 90)), (-2.0, -0.5), 1.0)
+    gpu = _capi.nwa_forward_marginals(s.to(cuda), None, go, ge, T)
     torch.cuda.synchronize()
-    _check(gpu, s.numpy(), -2.0, -0.5, 1.0)
+    _check(gpu, s.numpy(), go, ge, T)
 
 
-def test_nwa_split_ragged(cuda, parts):
+@pytest.mark.parametrize("sweeps", SWEEPS)
+def test_nwa_split_ragged(cuda, parts, sweeps):
     parts(4)
-    s = _seeded(40, (5, 700, 110))
+    s, (go, ge), T = in_units(sweeps, _seeded(40, (5, 700, 110)), (-2.0, -0.5), 0.7)
     lens = [[700, 110], [0, 40], [193, 0], [1, 1], [257, 81]]
     gpu = _capi.nwa_forward_marginals(s.to(cuda), torch.tensor(lens, dtype=torch.int32).to(cuda),
-                                      -2.0, -0.5, 0.7)
+                                      go, ge, T)
     torch.cuda.synchronize()
-    _check(gpu, s.numpy(), -2.0, -0.5, 0.7, lens)
+    _check(gpu, s.numpy(), go, ge, T, lens)
 
 
 @pytest.mark.parametrize("n", [0, 1])

@@ -17,6 +17,7 @@ import torch
 
 import _capi
 from _paramgrad import check_param_grad
+from _sweeps import SWEEPS, in_units
 from oracle import oracle as O
 
 pytestmark = pytest.mark.gpu
@@ -61,9 +62,10 @@ CASES = [
 ]
 
 
+@pytest.mark.parametrize("sweeps", SWEEPS)
 @pytest.mark.parametrize("seed,B,L1,L2,go,ge,T", CASES)
-def test_affine_matches_oracle(cuda, seed, B, L1, L2, go, ge, T):
-    s = _seeded(seed, (B, L1, L2), 2.0)
+def test_affine_matches_oracle(cuda, seed, B, L1, L2, go, ge, T, sweeps):
+    s, (go, ge), T = in_units(sweeps, _seeded(seed, (B, L1, L2), 2.0), (go, ge), T)
     ref = O.get("oracle").soft_sw_affine(s.numpy(), go, ge, T)
     gpu = _capi.swa_forward_marginals(s.to(cuda), None, go, ge, T)
     _check(gpu, ref, s.numpy(), go, ge, T)

@@ -17,6 +17,7 @@ import torch
 
 import _capi
 from _paramgrad import check_param_grad
+from _sweeps import SWEEPS, in_units
 from oracle import oracle as O
 
 pytestmark = pytest.mark.gpu
@@ -65,9 +66,10 @@ CASES = [
 ]
 
 
+@pytest.mark.parametrize("sweeps", SWEEPS)
 @pytest.mark.parametrize("seed,B,L1,L2,gap,T", CASES)
-def test_sw_capi_matches_oracle(cuda, seed, B, L1, L2, gap, T):
-    s = _seeded(seed, (B, L1, L2))
+def test_sw_capi_matches_oracle(cuda, seed, B, L1, L2, gap, T, sweeps):
+    s, (gap,), T = in_units(sweeps, _seeded(seed, (B, L1, L2)), (gap,), T)
     ref = O.get("oracle").soft_sw(s.numpy(), gap, T)
     out = _capi.sw_forward_marginals(s.to(cuda), None, gap, T)
     torch.cuda.synchronize()

@@ -7,7 +7,8 @@ rows, the stripe above's last row and the scores.  The rebuilt rows must equal t
 stored ones, so every output equals the full-table form
 (D2P_AMD_SW_RECOMPUTE=0) bit for bit: full and ragged lengths, empty elements,
 rows shorter than a chunk, columns past the element, split parts, the
-allocation-free entry point, and the public op.  Each case is also held to the
+allocation-free entry point, and the public op.  All in units whose temperature the
+log-domain sweeps take (_sweeps.py): the linear-domain ones know no such switch.  Each case is also held to the
 oracle at the north-star tolerances (value 1e-5 relative, marginals 1e-4 absolute).
 """
 import numpy as np
@@ -15,6 +16,7 @@ import pytest
 import torch
 
 import _capi
+from _sweeps import assert_log_domain, in_units
 from oracle import oracle as O
 from test_gpu_sw_linear import _check, _seeded
 
@@ -22,6 +24,7 @@ pytestmark = pytest.mark.gpu
 
 
 def _both(monkeypatch, fn):
+    assert_log_domain(fn)
     out = {}
     for flag in ("1", "0"):
         monkeypatch.setenv("D2P_AMD_SW_RECOMPUTE", flag)
@@ -53,7 +56,7 @@ CASES = [
 def test_recompute_bit_identical_and_matches_oracle(cuda, monkeypatch, seed, B, L1, L2, n,
                                                     ragged):
     monkeypatch.setenv("D2P_AMD_SPLIT", str(n))
-    s = _seeded(seed, (B, L1, L2), 1.5)
+    s, (gap,), T = in_units("log domain", _seeded(seed, (B, L1, L2), 1.5), (-1.0,), 0.8)
     lengths = None
     if ragged:
         g = np.random.default_rng(seed)
@@ -63,13 +66,13 @@ def test_recompute_bit_identical_and_matches_oracle(cuda, monkeypatch, seed, B, 
         lengths[-1] = [0, L2]
     dl = None if lengths is None else torch.from_numpy(lengths).to(cuda)
     sd = s.to(cuda)
-    out = _both(monkeypatch, lambda: _capi.sw_forward_marginals(sd, dl, -1.0, 0.8))
-    ref = O.get("oracle").soft_sw(s.numpy(), -1.0, 0.8, lengths)
-    _check(out, ref, lengths=lengths, gap=-1.0, T=0.8, scores=s.numpy())
+    out = _both(monkeypatch, lambda: _capi.sw_forward_marginals(sd, dl, gap, T))
+    ref = O.get("oracle").soft_sw(s.numpy(), gap, T, lengths)
+    _check(out, ref, lengths=lengths, gap=gap, T=T, scores=s.numpy())
 
 
 def test_recompute_noalloc_entry(cuda, monkeypatch):
-    s = _seeded(67, (8, 512, 384)).to(cuda)
+    s, (gap,), T = in_units("log domain", _seeded(67, (8, 512, 384)).to(cuda), (-1.0,), 1.0)
     B, L1, L2 = s.shape
     lens = torch.tensor([[L1, L2]] * B, dtype=torch.int32, device=cuda)
 
@@ -77,7 +80,7 @@ def test_recompute_noalloc_entry(cuda, monkeypatch):
         outs = [torch.full((B,), 7.0, device=cuda), torch.full((B, L1, L2), 7.0, device=cuda),
                 torch.full((B,), 7.0, device=cuda), torch.full((B,), 7.0, device=cuda)]
         _capi.check(_capi.lib().d2p_sw_forward_marginals_noalloc(
-            _capi.ptr(s), _capi.ptr(lens), B, L1, L2, -1.0, 1.0,
+            _capi.ptr(s), _capi.ptr(lens), B, L1, L2, gap, T,
             *[_capi.ptr(o) for o in outs], _capi.stream()))
         return outs
     _both(monkeypatch, run)
@@ -85,11 +88,11 @@ def test_recompute_noalloc_entry(cuda, monkeypatch):
 
 def test_recompute_public_op(cuda, monkeypatch):
     import d2p_amd
-    s = _seeded(68, (6, 400, 300)).to(cuda)
+    s, (gap,), T = in_units("log domain", _seeded(68, (6, 400, 300)).to(cuda), (-1.0,), 1.0)
 
     def run():
         x = s.clone().requires_grad_(True)
-        r = d2p_amd.soft_sw(x, gap=-1.0, temperature=1.0)
+        r = d2p_amd.soft_sw(x, gap=gap, temperature=T)
         r.value.sum().backward()
         return [r.value.detach(), r.marginals.detach(), x.grad]
     _both(monkeypatch, run)

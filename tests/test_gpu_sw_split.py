@@ -7,7 +7,8 @@ D2P_AMD_SPLIT=<n> forces n parts per element (1: never split); unset, the librar
 splits only long elements of small batches.  Every case is checked against the CPU
 oracle to the north-star tolerances (value 1e-5 relative, marginals 1e-4
 absolute, parameter gradients as in test_gpu_sw_linear), with the pipeline status
-words required to stay 0 (no wait ran into its bound).  The HVP case checks that
+words required to stay 0 (no wait ran into its bound).  The first-order cases run
+through either kind of sweeps that takes them (_sweeps.py).  The HVP case checks that
 the second-order entry points (primal sweeps, tangent sweep and two-channel reverse
 sweep all split) stay within 1e-4 * max(1, max|H|), and the Jacobians and the
 marginal-path backward within the allowances of test_gpu_sw_second.
@@ -17,6 +18,7 @@ import pytest
 import torch
 
 import _capi
+from _sweeps import SWEEPS, assert_log_domain, in_units
 from oracle import oracle as O
 from test_gpu_sw_linear import _check, _seeded
 from test_gpu_sw_second import _close, _jacobian_ref
@@ -45,22 +47,24 @@ CASES = [
 ]
 
 
+@pytest.mark.parametrize("sweeps", SWEEPS)
 @pytest.mark.parametrize("seed,B,L1,L2,n", CASES)
-def test_sw_split_matches_oracle(cuda, parts, seed, B, L1, L2, n):
+def test_sw_split_matches_oracle(cuda, parts, seed, B, L1, L2, n, sweeps):
     parts(n)
-    s = _seeded(seed, (B, L1, L2))
-    ref = O.get("oracle").soft_sw(s.numpy(), -1.0, 1.0)
-    out = _capi.sw_forward_marginals(s.to(cuda), None, -1.0, 1.0)
+    s, (gap,), T = in_units(sweeps, _seeded(seed, (B, L1, L2)), (-1.0,), 1.0)
+    ref = O.get("oracle").soft_sw(s.numpy(), gap, T)
+    out = _capi.sw_forward_marginals(s.to(cuda), None, gap, T)
     torch.cuda.synchronize()
-    _check(out, ref, scores=s.numpy())
+    _check(out, ref, gap=gap, T=T, scores=s.numpy())
 
 
-def test_sw_split_ragged(cuda, parts):
+@pytest.mark.parametrize("sweeps", SWEEPS)
+def test_sw_split_ragged(cuda, parts, sweeps):
     """Ragged lengths under 4 parts of 3 stripes: elements whose later parts hold no
     stripe, empty elements, and one-row elements."""
     parts(4)
     B, L1, L2 = 7, 700, 170
-    s = _seeded(29, (B, L1, L2), 2.0)
+    s, (gap,), T = in_units(sweeps, _seeded(29, (B, L1, L2), 2.0), (-1.0,), 0.5)
     g = np.random.default_rng(29)
     lengths = np.stack([g.integers(0, L1 + 1, B), g.integers(0, L2 + 1, B)], 1).astype(np.int32)
     lengths[0] = [L1, L2]
@@ -68,10 +72,10 @@ def test_sw_split_ragged(cuda, parts):
     lengths[2] = [640, 0]
     lengths[3] = [1, 1]
     lengths[4] = [193, 170]      # the first part only (stripes 0..3 of 11)
-    ref = O.get("oracle").soft_sw(s.numpy(), -1.0, 0.5, lengths)
-    out = _capi.sw_forward_marginals(s.to(cuda), torch.from_numpy(lengths).to(cuda), -1.0, 0.5)
+    ref = O.get("oracle").soft_sw(s.numpy(), gap, T, lengths)
+    out = _capi.sw_forward_marginals(s.to(cuda), torch.from_numpy(lengths).to(cuda), gap, T)
     torch.cuda.synchronize()
-    _check(out, ref, lengths=lengths, gap=-1.0, T=0.5, scores=s.numpy())
+    _check(out, ref, lengths=lengths, gap=gap, T=T, scores=s.numpy())
 
 
 @pytest.mark.parametrize("B,L1,L2,n", [(2, 700, 260, 4), (3, 200, 300, 1), (1, 1500, 90, 8),
@@ -88,36 +92,43 @@ def test_sw_helper_waves_bit_identical(cuda, parts, monkeypatch, B, L1, L2, n):
     output equals the single-wave form
     bit for bit: SW and NW first order, the SW and NW HVPs, the SW parameter
     Jacobians, the marginal-path backward and affine SW first order, ragged lengths
-    and split parts included."""
-    s = _seeded(41, (B, L1, L2)).to(cuda)
+    and split parts included.  In units that the log-domain sweeps take: the
+    linear-domain ones know no such switch."""
+    s, (gap, go, ge), T = in_units("log domain", _seeded(41, (B, L1, L2)).to(cuda),
+                                   (-1.0, -3.0, -0.5), 0.9)
     lens = torch.tensor([[max(1, L1 - 37 * i), max(1, L2 - 11 * i)] for i in range(B)],
                         dtype=torch.int32, device=cuda)
     V = _seeded(42, (B, L1, L2)).to(cuda)
     parts(n)
+
+    def run():
+        return (list(_capi.sw_forward_marginals(s, lens, gap, T)) +
+                list(_capi.nw_forward_marginals(s, lens, gap, T)) +
+                [_capi.sw_hvp(s, V, lens, gap, T), _capi.nw_hvp(s, V, lens, gap, T),
+                 _capi.sw_param_jacobian(s, 0, lens, gap, T),
+                 _capi.sw_param_jacobian(s, 1, lens, gap, T)] +
+                list(_capi.sw_backward_full(s, V, lens, gap, T)) +
+                list(_capi.swa_forward_marginals(s, lens, go, ge, T)))
+    assert_log_domain(run)
     out = {}
     for flag in ("1", "0"):
         monkeypatch.setenv("D2P_AMD_SW_HELPERS", flag)
-        out[flag] = (list(_capi.sw_forward_marginals(s, lens, -1.0, 0.9)) +
-                     list(_capi.nw_forward_marginals(s, lens, -1.0, 0.9)) +
-                     [_capi.sw_hvp(s, V, lens, -1.0, 0.9), _capi.nw_hvp(s, V, lens, -1.0, 0.9),
-                      _capi.sw_param_jacobian(s, 0, lens, -1.0, 0.9),
-                      _capi.sw_param_jacobian(s, 1, lens, -1.0, 0.9)] +
-                     list(_capi.sw_backward_full(s, V, lens, -1.0, 0.9)) +
-                     list(_capi.swa_forward_marginals(s, lens, -3.0, -0.5, 0.9)))
+        out[flag] = run()
     for i, (a, b) in enumerate(zip(out["1"], out["0"])):
         assert torch.equal(a, b), f"output {i}: max |diff| {float((a - b).abs().max()):.3e}"
-    ref = O.get("oracle").soft_sw(s.cpu().numpy(), -1.0, 0.9, lens.cpu().numpy())
+    ref = O.get("oracle").soft_sw(s.cpu().numpy(), gap, T, lens.cpu().numpy())
     np.testing.assert_allclose(out["1"][0].cpu().numpy(), ref[0], rtol=1e-5, atol=1e-6)
 
 
-def test_sw_split_repeated_launches(cuda, parts):
+@pytest.mark.parametrize("sweeps", SWEEPS)
+def test_sw_split_repeated_launches(cuda, parts, sweeps):
     """Consecutive launches on one workspace: the progress words of one launch never
     satisfy the waits of the next (epochs), and the results repeat exactly."""
     parts(3)
-    s = _seeded(30, (2, 700, 120)).to(cuda)
-    first = _capi.sw_forward_marginals(s, None, -1.0, 1.0)
+    s, (gap,), T = in_units(sweeps, _seeded(30, (2, 700, 120)).to(cuda), (-1.0,), 1.0)
+    first = _capi.sw_forward_marginals(s, None, gap, T)
     for _ in range(3):
-        again = _capi.sw_forward_marginals(s, None, -1.0, 1.0)
+        again = _capi.sw_forward_marginals(s, None, gap, T)
         for a, b in zip(first, again):
             torch.testing.assert_close(a, b, rtol=0, atol=0)
 
@@ -183,23 +194,25 @@ AFFINE_CASES = [
 ]
 
 
+@pytest.mark.parametrize("sweeps", SWEEPS)
 @pytest.mark.parametrize("seed,B,L1,L2,go,ge,T,n", AFFINE_CASES)
-def test_affine_split_matches_oracle(cuda, parts, seed, B, L1, L2, go, ge, T, n):
+def test_affine_split_matches_oracle(cuda, parts, seed, B, L1, L2, go, ge, T, n, sweeps):
     from test_gpu_sw_affine import _check as _check_affine
     parts(n)
-    s = _seeded(seed, (B, L1, L2), 2.0)
+    s, (go, ge), T = in_units(sweeps, _seeded(seed, (B, L1, L2), 2.0), (go, ge), T)
     ref = O.get("oracle").soft_sw_affine(s.numpy(), go, ge, T)
     gpu = _capi.swa_forward_marginals(s.to(cuda), None, go, ge, T)
     torch.cuda.synchronize()
     _check_affine(gpu, ref, s.numpy(), go, ge, T)
 
 
-def test_affine_split_ragged(cuda, parts):
+@pytest.mark.parametrize("sweeps", SWEEPS)
+def test_affine_split_ragged(cuda, parts, sweeps):
     """Config C3 style lengths under 4 parts: elements whose later parts are empty."""
     from test_gpu_sw_affine import _check as _check_affine
     parts(4)
     B, L1, L2 = 6, 700, 260
-    s = _seeded(46, (B, L1, L2), 2.0)
+    s, (go, ge), T = in_units(sweeps, _seeded(46, (B, L1, L2), 2.0), (-11.0, -1.0), 0.5)
     g = torch.Generator().manual_seed(47)
     lens = torch.randint(64, L1 + 1, (B, 2), generator=g, dtype=torch.int32)
     lens[:, 1] = torch.clamp(lens[:, 1], max=L2)
@@ -207,10 +220,10 @@ def test_affine_split_ragged(cuda, parts):
     lens[2] = torch.tensor([640, 0])
     lens[3] = torch.tensor([L1, L2])
     lens[4] = torch.tensor([150, 260])
-    ref = O.get("oracle").soft_sw_affine(s.numpy(), -11.0, -1.0, 0.5, lens.numpy())
-    gpu = _capi.swa_forward_marginals(s.to(cuda), lens.to(cuda), -11.0, -1.0, 0.5)
+    ref = O.get("oracle").soft_sw_affine(s.numpy(), go, ge, T, lens.numpy())
+    gpu = _capi.swa_forward_marginals(s.to(cuda), lens.to(cuda), go, ge, T)
     torch.cuda.synchronize()
-    _check_affine(gpu, ref, s.numpy(), -11.0, -1.0, 0.5, lens.tolist())
+    _check_affine(gpu, ref, s.numpy(), go, ge, T, lens.tolist())
 
 
 @pytest.mark.parametrize("n", [2, 3, 11])
