@@ -276,16 +276,19 @@ __device__ __forceinline__ void post(int* prog, int wave, int value) {
     __asm__ volatile("" ::: "memory");
 }
 
-// Waits of a stripe's two waves on each other: as wait_for, bounded by the default spin
-// limit whatever the tests set for the waits between stripes and parts.
+// Waits of a stripe's own waves on each other: as wait_for, with shorter sleeps and without its
+// wait for this wave's own LDS operations, which execute in order.
 __device__ __forceinline__ void wait_own(int* prog, int w, int need, int* status_b) {
-    int spins = 0;
-    while (prog_load(prog, w) < need) {
-        __builtin_amdgcn_s_sleep(1);
-        if (++spins >= SPIN_LIMIT) {
-            atomicOr(status_b, 1);
-            break;
-        }
+    if (prog_load(prog, w) < need) {
+        const int limit = __builtin_amdgcn_readfirstlane(g_spin_limit);
+        int spins = 0;
+        do {
+            __builtin_amdgcn_s_sleep(1);
+            if (++spins >= limit) {
+                atomicOr(status_b, 1);
+                break;
+            }
+        } while (prog_load(prog, w) < need);
     }
     __asm__ volatile("" ::: "memory");
 }

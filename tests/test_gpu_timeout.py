@@ -19,6 +19,7 @@ import torch
 
 import d2p_amd
 from _capi import check, lib, ptr, stream
+from _sweeps import assert_log_domain, in_units
 from oracle import oracle as O
 
 pytestmark = pytest.mark.gpu
@@ -45,7 +46,7 @@ def _status_words(ws, B):
     return ws[:4 * B].view(torch.int32).cpu().numpy()
 
 
-def _sw_call(x, lengths, split=None):
+def _sw_call(x, lengths, split=None, gap=-1.0, T=1.0):
     B, L1, L2 = x.shape
     dev = x.device
     outs = [torch.empty(B, device=dev), torch.empty(B, L1, L2, device=dev),
@@ -56,7 +57,7 @@ def _sw_call(x, lengths, split=None):
     if split is not None:
         os.environ["D2P_AMD_SPLIT"] = str(split)
     try:
-        check(lib().d2p_sw_forward_marginals(ptr(x), ptr(lengths), B, L1, L2, -1.0, 1.0,
+        check(lib().d2p_sw_forward_marginals(ptr(x), ptr(lengths), B, L1, L2, gap, T,
                                              *[ptr(o) for o in outs], ptr(ws), n, stream()))
     finally:
         if split is not None:
@@ -88,12 +89,14 @@ def test_sw_forward_marginals_gives_up_to_nan(cuda, low_spin_limit, monkeypatch,
     # element never waits; with them (parts of at most four stripes: both split
     # settings here) its sweeping wave and its helper wait on each other, so it may be
     # marked too.
+    # (in units that the log-domain sweeps take, which know the switch)
     monkeypatch.setenv("D2P_AMD_SW_HELPERS", helpers)
-    s = _scores(3, 330, 150, 41)
+    s, (gap,), T = in_units("log domain", _scores(3, 330, 150, 41), (-1.0,), 1.0)
     lengths = torch.tensor([[50, 150], [330, 150], [260, 120]], dtype=torch.int32)
-    part, post, _, _ = O.get("oracle").soft_sw(s.numpy(), -1.0, 1.0, lengths.numpy())
+    part, post, _, _ = O.get("oracle").soft_sw(s.numpy(), gap, T, lengths.numpy())
     x, ln = s.to(cuda), lengths.to(cuda)
-    outs, ws = _sw_call(x, ln, split)
+    assert_log_domain(lambda: _sw_call(x, ln, split, gap, T))
+    outs, ws = _sw_call(x, ln, split, gap, T)
     status = _status_words(ws, 3)
     assert status[1] != 0 and status[2] != 0
     if helpers == "0":
@@ -102,6 +105,30 @@ def test_sw_forward_marginals_gives_up_to_nan(cuda, low_spin_limit, monkeypatch,
     st = ctypes.c_int(0)
     check(lib().d2p_sw_status(ptr(ws), 3, ctypes.byref(st), stream()))
     assert st.value != 0
+
+
+@pytest.mark.parametrize("split", [None, 3])
+@pytest.mark.parametrize("B,redone", [(3, False), (3, True), (300, False)])
+def test_linear_domain_sweeps_give_up_to_nan(cuda, low_spin_limit, split, B, redone):
+    """Both launch shapes, and with elements that the log-domain sweeps redo."""
+    s = _scores(B, 330, 150, 41)
+    if redone:
+        s[1, 3, 4] = 300.0
+    lengths = torch.tensor([[50, 150], [330, 150], [260, 120]] * (B // 3), dtype=torch.int32)
+    part, post, _, _ = O.get("oracle").soft_sw(s[:3].numpy(), -1.0, 1.0, lengths[:3].numpy())
+    outs, ws = _sw_call(s.to(cuda), lengths.to(cuda), split)
+    status = _status_words(ws, B)
+    assert status[1] != 0 and status[2] != 0
+    _assert_contract([o[:3] for o in outs], status[:3], (part, post))
+
+
+def test_waits_within_a_stripe_give_up_to_nan(cuda, low_spin_limit):
+    """Elements of one stripe, whose sweeping and helper waves wait for each other only."""
+    s = _scores(3, 50, 150, 46)
+    part, post, _, _ = O.get("oracle").soft_sw(s.numpy(), -1.0, 1.0)
+    lengths = torch.tensor([[50, 150]] * 3, dtype=torch.int32, device=cuda)
+    outs, ws = _sw_call(s.to(cuda), lengths)
+    _assert_contract(outs, _status_words(ws, 3), (part, post))
 
 
 def test_second_order_and_other_families_give_up_to_nan(cuda, low_spin_limit):
