@@ -1635,8 +1635,7 @@ int launch_forward_k(const float* scores, const int* lengths, int B, int max_L1,
     const int ns = (max_L1 + 63) / 64;
     D2P_HIP(hipFuncSetAttribute((const void*)sw_forward_kernel<NWG, HELP, WIDE, TAN>,
                                 hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
-    // (labelled as the tangent sweep that it takes the place of)
-    D2P_LAUNCH(TAN ? (NWG ? "nw_tangent" : "sw_tangent")
+    D2P_LAUNCH(TAN ? (NWG ? "nw_forward_tangent" : "sw_forward_tangent")
                    : (NWG ? "nw_forward" : "sw_forward"),
                (sw_forward_kernel<NWG, HELP, WIDE, TAN>),
                dim3(wf::split_grid(B, sp.G)), dim3((WIDE ? 2 : 1) * wf::NW * 64), lds, st, scores,

@@ -168,8 +168,8 @@ def _kernels_launched(fn):
     return {line.split()[0] for line in buf.value.decode().splitlines()}
 
 
-SECOND_ORDER = ("sw_tangent", "sw_dual", "nw_tangent", "nw_dual", "swa_tangent", "swa_dual",
-                "nwa_tangent", "nwa_dual",
+SECOND_ORDER = ("sw_tangent", "sw_forward_tangent", "sw_dual", "nw_tangent", "nw_forward_tangent",
+                "nw_dual", "swa_tangent", "swa_dual", "nwa_tangent", "nwa_dual",
                 "dtw_tangent", "dtw_dual")
 
 
@@ -198,7 +198,9 @@ def test_value_path_launches_no_second_order_kernels(cuda, family):
     assert not names & set(SECOND_ORDER), names
     names = _kernels_launched(marginal_path)
     prefix = {"sw": "sw", "swa": "swa", "dtw": "dtw", "nw": "nw", "nwa": "nwa"}[family]
-    assert {f"{prefix}_tangent", f"{prefix}_dual"} <= names, names
+    # (linear gaps: the tangent rides on the forward)
+    tangent = f"{prefix}_forward_tangent" if family in ("sw", "nw") else f"{prefix}_tangent"
+    assert {tangent, f"{prefix}_dual"} <= names, names
 
 
 def test_null_lengths_mean_full_lengths(cuda):
