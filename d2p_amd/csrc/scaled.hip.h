@@ -13,7 +13,9 @@
 // and the marginal is P = E (a[i-1,j-1] + 1) b / Z.  The forward keeps one checkpoint per
 // 16-step chunk (the state that enters it) instead of a table, and the reverse sweep
 // rebuilds the chunk's values from it in registers, in the scale that makes a b / Z the
-// marginal itself.  Sums are in 64 bits throughout: only E carries a 32-bit rounding.
+// marginal itself.  E carries a 32-bit rounding; values, flows and gap sums are in 64 bits;
+// the sum of P s takes P as it is stored, in 32 bits, and is in 32 bits over the 16 steps of a
+// chunk (with helper waves it takes s from E, log2 E / c) and in 64 bits beyond.
 //
 // Range.  Scores that move a lane's values up by more than about 60 bits a step take them
 // beyond 2^1023 of its chunk's scale: they become infinite or NaN, which the sweeps detect.
@@ -141,7 +143,6 @@ struct Args {
     float* gradT;
     int* status;
     int* redo;
-    float* trash;
     uint64_t* fflag;
     uint64_t* bflag;
     double* bpart;        // [B][part][4]
@@ -300,7 +301,7 @@ __device__ __forceinline__ void wait_own(int* prog, int w, int need, int* status
 // t1: the diagonal sum; the marginal is t1 E b / Z.
 template <Fam F>
 struct FwdIn {
-    double f, gf, of;   // 2^(K_above - K), and times the gap / open factor
+    double f, gf;       // 2^(K_above - K), and (linear gaps) times the gap factor
     double one;         // the restart term in this lane's scale
 };
 

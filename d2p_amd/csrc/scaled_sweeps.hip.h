@@ -319,7 +319,6 @@ __global__ void __launch_bounds__(MAXW * 64) fwd_kernel(const Args A) {
             K = Kn;
             FwdIn<F> in;
             in.f = scale2(1.0, shr1(Kn, kr) - Kn);
-            in.gf = A.k.g * in.f;
             in.one = Tr::LOCAL ? scale2(1.0, -Kn) : 0.0;
 
             // checkpoint: the state that enters the chunk
@@ -1191,7 +1190,7 @@ __device__ __forceinline__ void fwd2_sweep(const Args& A, int b, int part) {
             const int ex = exponent(v);
             int Kn = K + (ex > -1023 && ex < 1024 ? ex : 0);
             if (Tr::LOCAL) Kn = max(Kn, kMinExp);
-            if (F != NW && k < 64 / P) {
+            if (Tr::LOCAL && k < 64 / P) {
                 const int kb = k == 0 ? kr : __builtin_amdgcn_readlane(Kn, max(k * P - 1, 0));
                 if (lane >= k * P) Kn = kb;
             }
@@ -1206,7 +1205,7 @@ __device__ __forceinline__ void fwd2_sweep(const Args& A, int b, int part) {
                 }
             }
             // (zeros from above the first stripe: any finite factor will do)
-            if (!ring_in && F != NW) kr = __builtin_amdgcn_readlane(Kn, 0);
+            if (!ring_in && Tr::LOCAL) kr = __builtin_amdgcn_readlane(Kn, 0);
             const int delta = K - Kn;
             v = scale2(v, delta);
             d = scale2(d, shr1(delta, kr_prev - kr));
@@ -1562,10 +1561,7 @@ __device__ __forceinline__ void bwd2_sweep(const Args& A, int b, int part) {
                     }
                     const bool ok = FULL || (unsigned)(t0 + j - lane) < lim;
                     const double wd = shl1(w, fl[(j / 4) & 1][j & 3]);
-                    double bn;
-                    if (F == SW) bn = __builtin_fma(A.k.g, bb, one);
-                    else if (F == NW) bn = A.k.g * bb;
-                    else bn = y;
+                    double bn = F == SW ? __builtin_fma(A.k.g, bb, one) : A.k.g * bb;
                     if (!FULL && F == NW && owns_end && t0 + j == t_end && lane == lane_end)
                         bn = scale2(1.0, -K);
                     bn = __builtin_fma(fb, wd, bn);
@@ -1649,7 +1645,7 @@ __device__ __forceinline__ void bwd2_sweep(const Args& A, int b, int part) {
                 if (lane > 0) d = scale2(d * invZ, su);
                 const int K_up = shr1(K, 0);         // (not inside the select: every lane active)
                 in.f = lane > 0 ? scale2(1.0, K - K_up) : scale2(invZ, ka4 + K - zk);
-                if (F != NW && !above && lane == 0) in.f = 0.0;
+                if (Tr::LOCAL && !above && lane == 0) in.f = 0.0;
                 in.gf = A.k.g * in.f;
                 in.one = Tr::LOCAL ? scale2(invZ, K - zk) : 0.0;
             }

@@ -24,7 +24,6 @@ int run_scaled(const float* scores, const int* lengths, int B, int max_L1, int m
     A.gradT = grad_T;
     A.status = ws.status;
     A.redo = ws.redo;
-    A.trash = ws.trash;
     A.fflag = ws.fflag;
     A.bflag = ws.bflag;
     A.bpart = ws.bpart;
