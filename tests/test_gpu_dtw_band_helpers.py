@@ -7,6 +7,7 @@ import pytest
 import torch
 
 import d2p_amd
+from oracle import oracle as O
 
 pytestmark = pytest.mark.gpu
 
@@ -35,3 +36,20 @@ def test_banded_helpers_bit_identical(cuda, monkeypatch, B, L1, L2, band, parts,
         out[flag] = [t.clone() for t in d2p_amd.soft_dtw_with_grads(c, 0.5, lengths, band)]
     for a, b in zip(out["1"], out["0"]):
         assert torch.equal(a, b)
+
+
+@pytest.mark.parametrize("helpers", ["0", "1"])
+@pytest.mark.parametrize("L1,L2", [(1, 1), (1, 40), (40, 1), (33, 40), (40, 33), (7, 70), (129, 9),
+                                   (66, 13), (64, 16), (20, 131)])
+@pytest.mark.parametrize("band", [0, 1, 2, 5, 16, 1000])
+def test_marginals_are_positive_in_the_band_alone(cuda, monkeypatch, L1, L2, band, helpers):
+    # all paths alike: a cell's marginal is its share of the paths, 0 off the band
+    # (|j - i L2 / L1| <= bandwidth in 32-bit arithmetic, as the oracle has it) and where no path
+    # inside it passes
+    monkeypatch.setenv("D2P_AMD_DTW_HELPERS", helpers)
+    c = np.zeros((2, L1, L2), np.float32)
+    want = O.get("oracle64").soft_dtw(c[:1].astype(np.float64), 1.0, None, band)[1]
+    assert not ((want > 0) & (want < 1e-30)).any()
+    torch.full((2, L1, L2), 7.0, device=cuda)
+    got = d2p_amd.soft_dtw_with_grads(torch.from_numpy(c).to(cuda), 1.0, None, band)[1]
+    assert np.array_equal(got.cpu().numpy() > 0, np.broadcast_to(want > 0, c.shape))
