@@ -324,7 +324,7 @@ def measured_valu(kernel, config):
     """VALUBusy (%) of each kernel from a committed rocprofv3 SQ-counter summary,
     profiles/<family>_<config>_valu.md (family = the kernel's prefix, sw or swa), if
     present: the table row ``| VALUBusy (%) | ... |`` under a header naming each
-    kernel in backticks.  Returns {kernel short name: percent} or None."""
+    kernel, or its launch label, in backticks.  Returns {kernel short name: percent} or None."""
     path = os.path.join(ROOT, "profiles", f"{kernel.split('_')[0]}_{config}_valu.md")
     if not os.path.exists(path):
         return None
