@@ -183,8 +183,8 @@ struct OnlineLSEDot {
     }
 };
 
-template <typename Op>
-__device__ __forceinline__ float wave_reduce(float v, Op op) {
+template <typename T, typename Op>
+__device__ __forceinline__ T wave_reduce(T v, Op op) {
 #pragma unroll
     for (int off = 32; off >= 1; off >>= 1) v = op(v, __shfl_xor(v, off, 64));
     return v;

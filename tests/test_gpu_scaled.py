@@ -227,6 +227,18 @@ def test_strong_scores(cuda, B, L1, L2, T, op):
     _check([x[:4] for x in got], want, s[:4], (-1.0,), T, tol, op == "soft_nw")
 
 
+@pytest.mark.parametrize("L2", range(189, 206))
+@pytest.mark.parametrize("op,gaps", [("soft_nw", (-2.5,)), ("soft_nw_affine", (-3.0, -2.5))])
+def test_values_far_below_their_chunk(cuda, op, gaps, L2):
+    # the element ends on a run of gaps, 14 bits each: its value lies up to 16 of them below the
+    # exponent that its chunk began with, through the end of the 32-bit range
+    s, _ = _inputs(2, 100, L2, False)
+    s[:, :, 100:] -= 20.0
+    got = getattr(d2p_amd, op + "_with_grads")(torch.from_numpy(s).to(cuda), *gaps, 0.25, None)
+    want = getattr(O.get("oracle64"), op)(s.astype(np.float64), *gaps, 0.25, None)
+    _check(got, want, s, gaps, 0.25, _tol(s, 100, 0.25), True)
+
+
 def _segments(L1, L2, T, match, penalty):
     """Matches along the diagonal, everything else and the diagonal's middle cell at the
     penalty: (local alignment, affine gaps) one path has both halves, through that cell."""
