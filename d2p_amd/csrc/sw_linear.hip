@@ -1154,8 +1154,20 @@ __device__ __forceinline__ void backward_sweep(const float* __restrict__ scores,
             for (int j = 0; j < P; ++j) A[j + 2] = buf[ABUF + rows_row<P, -1>(j) * 64 + lane];
             // lane j: alpha of the row above at lane-63 step t_hi - j + 63 (column
             // t_hi - j); above the first stripe, row 0: NINF, or (NWG) (column + 1) * gap
-            // FULL: every cell of the chunk lies inside the element
-            const bool inside = i0 + 63 < L1 && t_hi - P - 62 >= 0 && t_hi < L2;
+            // FULL: every cell of the chunk lies inside the element (SW: and none of their
+            // alphas is so low, behind a mask, that the rounding of alpha c, 2^-24 of it,
+            // leaves the range of 2^x: the other form takes differences first)
+            bool inside = i0 + 63 < L1 && t_hi - P - 62 >= 0 && t_hi < L2;
+            if (!NWG && inside) {
+                // (a row's alphas fall by a gap a column at most: the first column tells
+                // for the chunk, but for gaps of that size themselves)
+                float amin = A[P - 1];
+                if (gap * c < -1048576.0f) {
+#pragma unroll
+                    for (int u = 0; u < P - 1; ++u) amin = fminf(amin, A[u]);
+                }
+                inside = __builtin_amdgcn_ballot_w64(amin * c < -536870912.0f) == 0;
+            }
             const bool bcast = BCAST && inside;
             float bv = 0.0f;
             // Contributions from the stripe below for lane 63.  The producer (lane 0 of
@@ -1302,11 +1314,16 @@ __device__ __forceinline__ void backward_sweep(const float* __restrict__ scores,
                 // PRECISE keeps the max: its registers are all in use.)
                 const float m = (FULL && !PRECISE) ? a0
                                 : NWG ? fmaxf(fmaxf(vd, vu), fmaxf(vl, -1e20f))
-                                      : fmaxf(fmaxf(vd, vu), fmaxf(fmaxf(vl, sc), -1e20f));
+                                      : fmaxf(fmaxf(vd, vu), fmaxf(vl, sc));
+                // (SW, not FULL: cells behind a mask, all of whose candidates are as low as
+                // its scores: differences, which are exact where it matters.)
+                constexpr bool DIFF = !NWG && !FULL;
                 const float mc = m * c;
-                const float e0 = fast_exp2(fmaf(vd, c, -mc)), e1 = fast_exp2(fmaf(vu, c, -mc));
-                const float e2 = fast_exp2(fmaf(vl, c, -mc));
-                const float e3 = NWG ? 0.0f : fast_exp2(fmaf(sc, c, -mc));
+                auto weight = [&](float v) {
+                    return fast_exp2(DIFF ? (v - m) * c : fmaf(v, c, -mc));
+                };
+                const float e0 = weight(vd), e1 = weight(vu), e2 = weight(vl);
+                const float e3 = NWG ? 0.0f : weight(sc);
                 const float e03 = e0 + e3, e12 = e1 + e2;
                 const float rin = fast_rcp(e12 + e03);
                 float binit;

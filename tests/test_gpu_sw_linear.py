@@ -76,6 +76,24 @@ def test_sw_capi_matches_oracle(cuda, seed, B, L1, L2, gap, T, sweeps):
     _check(out, ref, gap=gap, T=T, scores=s.numpy())
 
 
+@pytest.mark.parametrize("masked", [-1e3, -1e9, -1e30])
+@pytest.mark.parametrize("B,L1,L2,T", [(2, 130, 70, 0.19), (2, 300, 83, 0.1), (3, 500, 200, 0.19),
+                                       (1, 1100, 1100, 1.0), (1, 1100, 2500, 1.0)])
+def test_sw_rows_and_columns_masked_from_the_start(cuda, B, L1, L2, T, masked):
+    """Cells behind a mask, whose alpha is the mask's own score: no marginal, and no NaN from
+    weights of such numbers; their parameter gradients and Jacobians as well."""
+    s = _seeded(70, (B, L1, L2), T)
+    s[:, :, :40] = masked
+    s[:, :20] = masked
+    ref = O.get("oracle").soft_sw(s.numpy(), -T, T)
+    out = _capi.sw_forward_marginals(s.to(cuda), None, -T, T)
+    torch.cuda.synchronize()
+    _check(out, ref, gap=-T, T=T, scores=s.numpy())
+    if L1 <= 300:
+        for p in (0, 1):
+            assert not torch.isnan(_capi.sw_param_jacobian(s.to(cuda), p, None, -T, T)).any()
+
+
 def test_sw_capi_ragged_lengths(cuda):
     B, L1, L2 = 7, 150, 170
     s = _seeded(11, (B, L1, L2), 2.0)
