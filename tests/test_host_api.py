@@ -34,7 +34,8 @@ def reference_schemas():
     return out
 
 
-@pytest.mark.skipif(not os.path.isdir(REF), reason="reference sources absent")
+@pytest.mark.skipif(not os.path.isdir(os.path.join(REF, "src")),
+                    reason="reference sources absent")
 def test_schemas_byte_identical_to_reference():
     ref = reference_schemas()
     assert len(ref) == 60   # 13 linear SW + 14 affine SW + 6 DTW + 13 linear NW + 14 affine NW
